@@ -21,6 +21,7 @@
 //                     C[m + M n], which is already the reference's C layout
 //                     (A's free axes low, B's high: src/Network.h:739-769).
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 
 #include "qt_internal.h"
@@ -319,39 +320,45 @@ __global__ __launch_bounds__(kThreads) void k_thin(const V* __restrict__ X, cons
     }
 }
 
-// Split reduction for outputs of at most kReduceMaxOut elements.  Block b sums the
-// summed-index chunk [b*chunk, (b+1)*chunk) for every output and writes
-// partials[b * nC + c]; k_reduce_final adds the partials in block order.
-constexpr int kReduceMaxOut = 64;
+// Long sums into few outputs (see reduce_shape): the summed index is split over lanes,
+// steps and workgroups, the outputs over row groups.
 constexpr int64_t kReduceMaxBlocks = int64_t(1) << 15;
 
 template <class V>
-__device__ __forceinline__ V shfl_down_v(V v, int d) {
+__device__ __forceinline__ V shfl_xor_v(V v, int d) {
     V r;
-    r.x = __shfl_down(v.x, d, 64);
-    r.y = __shfl_down(v.y, d, 64);
+    r.x = __shfl_xor(v.x, d, 64);
+    r.y = __shfl_xor(v.y, d, 64);
     return r;
 }
 
-// Rows of an operand: its elements that share one value of its free bits.  One pass of
-// k_reduce_rows reads GA rows of A and GB rows of B and accumulates the GA x GB outputs
-// they form, so an operand element is read once per pass, not once per output of the
-// other operand.  The summed index s splits into the lane (bits 0-7), the workgroup
-// (the next log2(gridDim.x) bits) and the step (the bits above), so the workgroups that
-// run together read neighbouring 256-element runs (with a contiguous chunk of s per
-// workgroup the kernel measured 2.7x slower on 2^24 summed indices).  Every output is
-// summed in the same order whatever the grouping: each lane over its steps in order,
-// then the lanes of a wave by shuffles, then the waves in order.
+// Rows of an operand: its elements that share one value of its free bits.  A workgroup
+// takes one group of GA rows of A and GB rows of B (blockIdx.y) and accumulates the
+// GA x GB outputs they form, so an operand element is read once per group of the other
+// side's rows.  The summed index s splits into the lane (bits 0-7), the workgroup (the
+// next log2(gridDim.x) bits) and the step (the bits above).  The host orders the summed
+// bits (order_summed_bits): the lanes of a wave cover the lowest summed bits of A and of
+// B in turn, so that both operands are read in whole 64-byte pieces however their axes
+// lie, and workgroups that run together read neighbouring runs.  Every output is summed
+// in the same order whatever the grouping: each lane over its steps in order, then the
+// lanes of a wave pairwise (lane bits 5 to 0), then the waves in order.
+// Bound by HBM.  A step of two complex64 operands (2^25 and 2^24 elements, shuffled axes,
+// 8 x 4 outputs, 2^22 summed indices: 403 MB), read-back included: 119 us, 586 us with
+// the lanes on the pairs' own bit order and two passes of 4 x 4 outputs.
 struct RowSet {
-    int64_t oa[16], ob[16];  // free-bit offsets of the pass's rows of A and of B
-    int16_t c[16];           // output index of row pair (i, j) at c[i * GB + j]
+    int64_t oa[32], ob[32];        // offsets of a group's rows of A and of B
+    int32_t c[32];                 // output offset of row pair (i, j) at c[i * GB + j]
+    int32_t n_ga, n_gb;            // group bits of A and of B (the group index is A's low, B's high)
+    int32_t ga_pos[24], ga_c[24];  // operand and output bit of each group bit of A
+    int32_t gb_pos[24], gb_c[24];
 };
 
 template <class V, int MODE, int GA, int GB>
 __global__ __launch_bounds__(kThreads) void k_reduce_rows(const V* __restrict__ A, const V* __restrict__ B,
-                                                          V* __restrict__ partials, BitMap m, int64_t nC,
-                                                          int step_bits, RowSet r) {
-    __shared__ V wsum[GA * GB][kThreads / 64];
+                                                          V* __restrict__ partials, BitMap m, int step_bits,
+                                                          RowSet r) {
+    constexpr int Q = GA * GB;
+    __shared__ V wsum[Q][kThreads / 64];
     // offsets of the step bits 0-5 and 6-11: plan bytes read inside the step loop
     // would be vector loads whose waits also wait for every operand load in flight
     __shared__ int64_t t_lo[2][64], t_hi[2][64];
@@ -359,6 +366,7 @@ __global__ __launch_bounds__(kThreads) void k_reduce_rows(const V* __restrict__ 
     const int lane = tid & 63, wave = tid >> 6;
     const int first_step_bit = m.nbits_s - step_bits;  // 8 + log2(gridDim.x)
     int64_t la = 0, lb = 0;
+#pragma unroll
     for (int j = 0; j < 8; ++j)
         if ((tid >> j) & 1) {
             la += int64_t(1) << m.s_a[j];
@@ -380,18 +388,28 @@ __global__ __launch_bounds__(kThreads) void k_reduce_rows(const V* __restrict__ 
             t_hi[1][x] = ob;
         }
     }
-    int64_t base_a = la, base_b = lb;  // lane and workgroup bits
+    int64_t base_a = la, base_b = lb;  // lane, workgroup and row-group bits
     for (int j = 8; j < first_step_bit; ++j)
         if ((blockIdx.x >> (j - 8)) & 1) {
             base_a += int64_t(1) << m.s_a[j];
             base_b += int64_t(1) << m.s_b[j];
         }
+    int64_t c0 = 0;
+    for (int i = 0; i < r.n_ga; ++i)
+        if ((blockIdx.y >> i) & 1) {
+            base_a += int64_t(1) << r.ga_pos[i];
+            c0 += int64_t(1) << r.ga_c[i];
+        }
+    for (int i = 0; i < r.n_gb; ++i)
+        if ((blockIdx.y >> (r.n_ga + i)) & 1) {
+            base_b += int64_t(1) << r.gb_pos[i];
+            c0 += int64_t(1) << r.gb_c[i];
+        }
     __syncthreads();
     Acc<V, MODE> acc[GA][GB];
-    // U steps per iteration, all loads issued before the first multiply (the steps are
-    // a power of two of at least 16, so U divides them).  Measured on 2^24 summed
-    // indices: 0.19 ms; with the U loads of an iteration on neighbouring runs instead
-    // of U steps apart, 0.60 ms
+    // U steps per iteration, all loads issued before the first multiply.  Measured on
+    // 2^24 summed indices: 0.19 ms; with the U loads of an iteration on neighbouring
+    // runs instead of U steps apart, 0.60 ms
     constexpr int U0 = GA + GB >= 16 ? 1 : 16 / (GA + GB);
     constexpr int U = U0 >= 8 ? 8 : U0 >= 4 ? 4 : U0 >= 2 ? 2 : 1;
     const int steps = 1 << step_bits;
@@ -400,6 +418,7 @@ __global__ __launch_bounds__(kThreads) void k_reduce_rows(const V* __restrict__ 
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int k = k0 + u;
+            if (u > 0 && k >= steps) break;  // fewer steps than U
             const int64_t ha = base_a + t_lo[0][k & 63] + t_hi[0][k >> 6];
             const int64_t hb = base_b + t_lo[1][k & 63] + t_hi[1][k >> 6];
 #pragma unroll
@@ -408,36 +427,57 @@ __global__ __launch_bounds__(kThreads) void k_reduce_rows(const V* __restrict__ 
             for (int j = 0; j < GB; ++j) b[u][j] = B[r.ob[j] + hb];
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < U; ++u) {
+            if (u > 0 && k0 + u >= steps) break;
 #pragma unroll
             for (int i = 0; i < GA; ++i)
 #pragma unroll
                 for (int j = 0; j < GB; ++j) mac<V, MODE>(acc[i][j], a[u][i], b[u][j]);
-    }
-#pragma unroll
-    for (int q = 0; q < GA * GB; ++q) {
-        V v = finish<V, MODE>(acc[q / GB][q % GB]);
-        for (int d = 32; d >= 1; d >>= 1) {
-            V o = shfl_down_v(v, d);
-            v.x += o.x;
-            v.y += o.y;
         }
-        if (lane == 0) wsum[q][wave] = v;
     }
+    // lanes pairwise at distances 32, 16, ..., 1.  While a lane holds more than one output
+    // it keeps the half that its lane bit names and hands the other half over; after
+    // log2(Q) distances it holds one output, whose index is its highest lane bits
+    V v[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) v[q] = finish<V, MODE>(acc[q / GB][q % GB]);
+    int q_own = 0;
+#pragma unroll
+    for (int l = 5; l >= 0; --l) {
+        const int d = 1 << l, done = 1 << (5 - l);  // outputs per lane: Q / done
+        if (Q / done > 1) {
+            const int half = Q / done / 2;
+            const bool up = (lane & d) != 0;
+#pragma unroll
+            for (int q = 0; q < half; ++q) {
+                const V keep = up ? v[q + half] : v[q], give = up ? v[q] : v[q + half];
+                const V got = shfl_xor_v(give, d);
+                v[q].x = keep.x + got.x;
+                v[q].y = keep.y + got.y;
+            }
+            if (up) q_own += half;
+        } else {
+            const V got = shfl_xor_v(v[0], d);
+            v[0].x += got.x;
+            v[0].y += got.y;
+        }
+    }
+    if ((lane & (64 / Q - 1)) == 0) wsum[q_own][wave] = v[0];
     __syncthreads();
-    if (tid < GA * GB) {
+    if (tid < Q) {
         V t = wsum[tid][0];
         for (int w = 1; w < kThreads / 64; ++w) {
             t.x += wsum[tid][w].x;
             t.y += wsum[tid][w].y;
         }
-        partials[int64_t(blockIdx.x) * nC + r.c[tid]] = t;
+        // one workgroup per output group: the result itself; else partials[c][workgroup]
+        partials[(c0 + r.c[tid]) * gridDim.x + blockIdx.x] = t;
     }
 }
 
 template <class V>
 __global__ __launch_bounds__(kThreads) void k_reduce_final(const V* __restrict__ partials, V* __restrict__ C,
-                                                           int64_t nC, int64_t nblocks) {
+                                                           int64_t nblocks) {
     // one workgroup per output: strided partial sums, then a fixed-shape tree (the
     // order does not depend on timing, so the result is reproducible)
     __shared__ V part[kThreads];
@@ -446,8 +486,9 @@ __global__ __launch_bounds__(kThreads) void k_reduce_final(const V* __restrict__
     t.x = 0;
     t.y = 0;
     for (int64_t b = threadIdx.x; b < nblocks; b += kThreads) {
-        t.x += partials[b * nC + c].x;
-        t.y += partials[b * nC + c].y;
+        const V p = partials[c * nblocks + b];
+        t.x += p.x;
+        t.y += p.y;
     }
     part[threadIdx.x] = t;
     __syncthreads();
@@ -982,114 +1023,159 @@ qt_status run_skinny(Ctx* c, const V* A, const V* B, V* C, const BitMap& m, int 
 }
 
 template <class V, int MODE, int GA, int GB>
-qt_status launch_rows(Ctx* c, dim3 grid, const V* A, const V* B, V* part, const BitMap& m, int64_t nC,
-                      int step_bits, const RowSet& r) {
-    hipLaunchKernelGGL((k_reduce_rows<V, MODE, GA, GB>), grid, dim3(kThreads), 0, c->stream, A, B, part, m, nC,
-                       step_bits, r);
+qt_status launch_rows(Ctx* c, dim3 grid, const V* A, const V* B, V* part, const BitMap& m, int step_bits,
+                      const RowSet& r) {
+    hipLaunchKernelGGL((k_reduce_rows<V, MODE, GA, GB>), grid, dim3(kThreads), 0, c->stream, A, B, part, m, step_bits,
+                       r);
     return check_hip(c, hipGetLastError(), "k_reduce_rows");
 }
 
 template <class V, int MODE>
 qt_status launch_reduce_rows(Ctx* c, int ga, int gb, dim3 grid, const V* A, const V* B, V* part, const BitMap& m,
-                             int64_t nC, int step_bits, const RowSet& r) {
-    switch (ga * 32 + gb) {
-        case 1 * 32 + 1: return launch_rows<V, MODE, 1, 1>(c, grid, A, B, part, m, nC, step_bits, r);
-        case 1 * 32 + 2: return launch_rows<V, MODE, 1, 2>(c, grid, A, B, part, m, nC, step_bits, r);
-        case 1 * 32 + 4: return launch_rows<V, MODE, 1, 4>(c, grid, A, B, part, m, nC, step_bits, r);
-        case 1 * 32 + 8: return launch_rows<V, MODE, 1, 8>(c, grid, A, B, part, m, nC, step_bits, r);
-        case 1 * 32 + 16: return launch_rows<V, MODE, 1, 16>(c, grid, A, B, part, m, nC, step_bits, r);
-        case 2 * 32 + 1: return launch_rows<V, MODE, 2, 1>(c, grid, A, B, part, m, nC, step_bits, r);
-        case 2 * 32 + 2: return launch_rows<V, MODE, 2, 2>(c, grid, A, B, part, m, nC, step_bits, r);
-        case 2 * 32 + 4: return launch_rows<V, MODE, 2, 4>(c, grid, A, B, part, m, nC, step_bits, r);
-        case 2 * 32 + 8: return launch_rows<V, MODE, 2, 8>(c, grid, A, B, part, m, nC, step_bits, r);
-        case 4 * 32 + 1: return launch_rows<V, MODE, 4, 1>(c, grid, A, B, part, m, nC, step_bits, r);
-        case 4 * 32 + 2: return launch_rows<V, MODE, 4, 2>(c, grid, A, B, part, m, nC, step_bits, r);
-        case 4 * 32 + 4: return launch_rows<V, MODE, 4, 4>(c, grid, A, B, part, m, nC, step_bits, r);
-        case 8 * 32 + 1: return launch_rows<V, MODE, 8, 1>(c, grid, A, B, part, m, nC, step_bits, r);
-        case 8 * 32 + 2: return launch_rows<V, MODE, 8, 2>(c, grid, A, B, part, m, nC, step_bits, r);
-        case 16 * 32 + 1: return launch_rows<V, MODE, 16, 1>(c, grid, A, B, part, m, nC, step_bits, r);
-        default: return set_error(c, QT_UNSUPPORTED, "split reduction: unsupported row grouping");
+                             int step_bits, const RowSet& r) {
+#define QT_ROWS(GA, GB) \
+    case GA * 64 + GB: return launch_rows<V, MODE, GA, GB>(c, grid, A, B, part, m, step_bits, r)
+    switch (ga * 64 + gb) {
+        QT_ROWS(1, 1); QT_ROWS(1, 2); QT_ROWS(1, 4); QT_ROWS(1, 8); QT_ROWS(1, 16);
+        QT_ROWS(2, 1); QT_ROWS(2, 2); QT_ROWS(2, 4); QT_ROWS(2, 8);
+        QT_ROWS(4, 1); QT_ROWS(4, 2); QT_ROWS(4, 4);
+        QT_ROWS(8, 1); QT_ROWS(8, 2);
+        QT_ROWS(16, 1);
+        default: break;
     }
+    if constexpr (sizeof(V) == 8) {
+        switch (ga * 64 + gb) {
+            QT_ROWS(1, 32); QT_ROWS(2, 16); QT_ROWS(4, 8); QT_ROWS(8, 4); QT_ROWS(16, 2); QT_ROWS(32, 1);
+            default: break;
+        }
+    }
+#undef QT_ROWS
+    return set_error(c, QT_UNSUPPORTED, "split reduction: unsupported row grouping");
+}
+
+// The summed bits in the order k_reduce_rows takes them: the lowest position in A not yet
+// taken, then the lowest in B, and so on (bits 0-5 are a wave's lanes: three bits of each
+// operand are 64 bytes of complex64, 128 of complex128).
+void order_summed_bits(BitMap& m) {
+    const int n = m.nbits_s;
+    int by_a[64], by_b[64];
+    for (int j = 0; j < n; ++j) by_a[j] = by_b[j] = j;
+    std::sort(by_a, by_a + n, [&](int x, int y) { return m.s_a[x] < m.s_a[y]; });
+    std::sort(by_b, by_b + n, [&](int x, int y) { return m.s_b[x] < m.s_b[y]; });
+    bool taken[64] = {false};
+    uint8_t sa[64], sb[64];
+    for (int k = 0, ia = 0, ib = 0; k < n; ++k) {
+        const int* by = (k & 1) == 0 ? by_a : by_b;
+        int& i = (k & 1) == 0 ? ia : ib;
+        while (taken[by[i]]) ++i;
+        const int j = by[i];
+        taken[j] = true;
+        sa[k] = m.s_a[j];
+        sb[k] = m.s_b[j];
+    }
+    std::memcpy(m.s_a, sa, size_t(n));
+    std::memcpy(m.s_b, sb, size_t(n));
 }
 
 template <class V, int MODE>
-qt_status run_reduce(Ctx* c, const V* A, const V* B, V* C, const BitMap& m, const Workspace* ws) {
+qt_status run_reduce(Ctx* c, const V* A, const V* B, V* C, const BitMap& m0, const Workspace* ws) {
+    BitMap m = m0;
+    order_summed_bits(m);
     const int64_t nC = int64_t(1) << m.nbits_c;
     const int64_t nS = int64_t(1) << m.nbits_s;
-    // each workgroup takes 16 steps of 256 summed indices, more only beyond 2^15
-    // workgroups, and at most 2^12 steps (k_reduce_rows' offset tables cover 12 step
-    // bits; nS >= 2^13 is a power of two, so the steps divide it)
-    int64_t chunk = kThreads * 16;
-    while (nS / chunk > kReduceMaxBlocks && chunk < (int64_t(1) << 20)) chunk <<= 1;
-    int step_bits = 0;
-    while ((int64_t(kThreads) << step_bits) < chunk) ++step_bits;
-    const int64_t nblocks = (nS + chunk - 1) / chunk;
-    const size_t need = size_t(nblocks * nC) * sizeof(V);
-    V* part = nullptr;
-    if (ws) {
-        if (need > ws->bytes) return set_error(c, QT_INVALID_INPUT, "split reduction: partial sums exceed the workspace");
-        part = reinterpret_cast<V*>(ws->base);
-    } else if (c->partials_bytes < need) {
-        if (c->partials) {
-            (void)hipStreamSynchronize(c->stream);
-            (void)hipFree(c->partials);
-            c->partials = nullptr;
-            c->partials_bytes = 0;
-        }
-        qt_status s = check_hip(c, hipMalloc(&c->partials, need), "partials");
-        if (s != QT_OK) return s;
-        c->partials_bytes = need;
+    // free bits of each side, lowest operand position first: a group's rows are the
+    // lowest ones, neighbours in memory
+    struct Bit {
+        int pos, c;
+    };
+    Bit fa[64], fb[64];
+    int ka = 0, kb = 0;
+    for (int i = 0; i < m.nbits_c; ++i) {
+        if (m.c_src[i] < 64) fa[ka++] = Bit{m.c_src[i], i};
+        else fb[kb++] = Bit{m.c_src[i] - 64, i};
     }
-    if (!part) part = static_cast<V*>(c->partials);
-    // rows: A's free bits enumerate na rows, B's nb rows; passes of ga x gb row pairs
-    // (at most 16 outputs per pass, so the accumulators stay in registers)
-    int64_t row_a[64], row_b[64];
-    int16_t c_of[64];
-    int na = 0, nb = 0;
-    {
-        int a_bits[6], b_bits[6], ka = 0, kb = 0;
-        for (int i = 0; i < m.nbits_c; ++i) {
-            if (m.c_src[i] < 64) a_bits[ka++] = i;
-            else b_bits[kb++] = i;
+    auto lower = [](const Bit& x, const Bit& y) { return x.pos < y.pos; };
+    std::sort(fa, fa + ka, lower);
+    std::sort(fb, fb + kb, lower);
+    // rows per group: A is read 2^(kb - gb) times, B 2^(ka - ga) times; the accumulators
+    // of 2^5 outputs (complex64) or 2^4 fit the registers at two waves per SIMD and more
+    const int out_bits = sizeof(V) == 8 ? 5 : 4;
+    int ga = 0, gb = 0;
+    double least = -1;
+    for (int x = 0; x <= ka && x <= out_bits; ++x) {
+        const int y = kb < out_bits - x ? kb : out_bits - x;
+        const double cost = std::ldexp(1.0, ka + kb - y) + std::ldexp(1.0, kb + ka - x);
+        if (least < 0 || cost < least) {
+            least = cost;
+            ga = x;
+            gb = y;
         }
-        na = 1 << ka;
-        nb = 1 << kb;
-        for (int x = 0; x < na; ++x) {
-            row_a[x] = 0;
-            for (int k = 0; k < ka; ++k)
-                if ((x >> k) & 1) row_a[x] += int64_t(1) << m.c_src[a_bits[k]];
+    }
+    const int64_t groups = int64_t(1) << (ka - ga + kb - gb);
+    // 16 steps of 256 summed indices per workgroup: fewer where that leaves the chip with
+    // less than two workgroups per CU (but not where it saves the second pass), more only
+    // beyond 2^15 workgroups, and at most 2^12 (the kernel's offset tables)
+    int step_bits = m.nbits_s - 8 < 4 ? m.nbits_s - 8 : 4;
+    while (step_bits > 0 && groups * ((nS >> 8) >> step_bits) < 512 && !(groups >= 128 && (nS >> 8) >> step_bits == 1))
+        --step_bits;
+    while ((nS >> 8) >> step_bits > kReduceMaxBlocks && step_bits < 12) ++step_bits;
+    // partial sums of at most 32 MiB
+    while (((nS >> 8) >> step_bits) * nC * int64_t(sizeof(V)) > (int64_t(32) << 20) && (nS >> 8) >> step_bits > 1 &&
+           step_bits < 12)
+        ++step_bits;
+    const int64_t nblocks = (nS >> 8) >> step_bits;
+    V* part = C;
+    if (nblocks > 1) {
+        const size_t need = size_t(nblocks * nC) * sizeof(V);
+        if (ws) {
+            if (need > ws->bytes)
+                return set_error(c, QT_INVALID_INPUT, "split reduction: partial sums exceed the workspace");
+            part = reinterpret_cast<V*>(ws->base);
+        } else {
+            if (c->partials_bytes < need) {
+                if (c->partials) {
+                    (void)hipStreamSynchronize(c->stream);
+                    (void)hipFree(c->partials);
+                    c->partials = nullptr;
+                    c->partials_bytes = 0;
+                }
+                qt_status s = check_hip(c, hipMalloc(&c->partials, need), "partials");
+                if (s != QT_OK) return s;
+                c->partials_bytes = need;
+            }
+            part = static_cast<V*>(c->partials);
         }
+    }
+    RowSet r;
+    std::memset(&r, 0, sizeof r);
+    const int na = 1 << ga, nb = 1 << gb;
+    for (int x = 0; x < na; ++x)
+        for (int k = 0; k < ga; ++k)
+            if ((x >> k) & 1) r.oa[x] += int64_t(1) << fa[k].pos;
+    for (int y = 0; y < nb; ++y)
+        for (int k = 0; k < gb; ++k)
+            if ((y >> k) & 1) r.ob[y] += int64_t(1) << fb[k].pos;
+    for (int x = 0; x < na; ++x)
         for (int y = 0; y < nb; ++y) {
-            row_b[y] = 0;
-            for (int k = 0; k < kb; ++k)
-                if ((y >> k) & 1) row_b[y] += int64_t(1) << (m.c_src[b_bits[k]] - 64);
+            int32_t o = 0;
+            for (int k = 0; k < ga; ++k)
+                if ((x >> k) & 1) o += 1 << fa[k].c;
+            for (int k = 0; k < gb; ++k)
+                if ((y >> k) & 1) o += 1 << fb[k].c;
+            r.c[x * nb + y] = o;
         }
-        for (int64_t cc = 0; cc < nC; ++cc) {
-            int x = 0, y = 0;
-            for (int k = 0; k < ka; ++k) x |= int((cc >> a_bits[k]) & 1) << k;
-            for (int k = 0; k < kb; ++k) y |= int((cc >> b_bits[k]) & 1) << k;
-            c_of[x * nb + y] = int16_t(cc);
-        }
+    for (int k = ga; k < ka; ++k, ++r.n_ga) {
+        r.ga_pos[r.n_ga] = fa[k].pos;
+        r.ga_c[r.n_ga] = fa[k].c;
     }
-    int ga = na < 16 ? na : 16, gb = nb < 16 ? nb : 16;
-    while (ga * gb > 16) {
-        if (ga >= gb) ga >>= 1;
-        else gb >>= 1;
+    for (int k = gb; k < kb; ++k, ++r.n_gb) {
+        r.gb_pos[r.n_gb] = fb[k].pos;
+        r.gb_c[r.n_gb] = fb[k].c;
     }
-    qt_status s = QT_OK;
-    for (int x0 = 0; x0 < na && s == QT_OK; x0 += ga)
-        for (int y0 = 0; y0 < nb && s == QT_OK; y0 += gb) {
-            RowSet r;
-            std::memset(&r, 0, sizeof r);
-            for (int i = 0; i < ga; ++i) r.oa[i] = row_a[x0 + i];
-            for (int j = 0; j < gb; ++j) r.ob[j] = row_b[y0 + j];
-            for (int i = 0; i < ga; ++i)
-                for (int j = 0; j < gb; ++j) r.c[i * gb + j] = c_of[(x0 + i) * nb + y0 + j];
-            s = launch_reduce_rows<V, MODE>(c, ga, gb, dim3(unsigned(nblocks)), A, B, part, m, nC, step_bits, r);
-        }
-    if (s != QT_OK) return s;
-
-    hipLaunchKernelGGL((k_reduce_final<V>), dim3(unsigned(nC)), dim3(kThreads), 0, c->stream, part, C, nC, nblocks);
+    qt_status s = launch_reduce_rows<V, MODE>(c, na, nb, dim3(unsigned(nblocks), unsigned(groups)), A, B, part, m,
+                                              step_bits, r);
+    if (s != QT_OK || nblocks == 1) return s;
+    hipLaunchKernelGGL((k_reduce_final<V>), dim3(unsigned(nC)), dim3(kThreads), 0, c->stream, part, C, nblocks);
     return check_hip(c, hipGetLastError(), "k_reduce_final");
 }
 
@@ -1673,15 +1759,23 @@ inline bool skinny_shape(const BitMap& m, bool split, int mbits) {
     return split && std::min(mbits, nbits_n) <= 5 && std::max(mbits, nbits_n) >= 10;
 }
 
+// Sums long enough to be split over a workgroup's lanes, into few outputs: from 2^9 summed
+// indices up to 2^11 outputs, from 2^11 up to 2^16.  k_direct and k_skinny run one lane
+// per output (or per 2 to 32 outputs), which leaves most of the chip idle there: 2^12
+// outputs over 2^12 summed indices (a state projected on 12 qubits, complex64) took
+// 1,244 us on k_skinny, 2^7 over 2^15 (complex128) 389 us on k_direct; here about 50 and
+// 20 us.
+inline bool reduce_shape(const BitMap& m) {
+    return (m.nbits_s >= 11 && m.nbits_c <= 16) || (m.nbits_s >= 9 && m.nbits_c <= 11);
+}
+
 template <class V, int MODE>
 qt_status dispatch_small(Ctx* c, const Tensor* A, const Tensor* B, Tensor* C, const BitMap& m, bool split,
                          int mbits, const Workspace* ws) {
     const V* a = static_cast<const V*>(A->data);
     const V* b = static_cast<const V*>(B->data);
     V* cc = static_cast<V*>(C->data);
-    const int64_t nC = int64_t(1) << m.nbits_c;
-    const int64_t nS = int64_t(1) << m.nbits_s;
-    if (nC <= kReduceMaxOut && nS >= 8192) return run_reduce<V, MODE>(c, a, b, cc, m, ws);
+    if (reduce_shape(m)) return run_reduce<V, MODE>(c, a, b, cc, m, ws);
     if (skinny_shape(m, split, mbits)) return run_skinny<V, MODE>(c, a, b, cc, m, mbits);
     return run_direct<V, MODE>(c, a, b, cc, m);
 }

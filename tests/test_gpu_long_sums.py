@@ -1,0 +1,55 @@
+"""Long sums into few outputs (k_reduce_rows) against numpy's tensordot in complex128
+(which pins the oracle's loop nest, tests/test_oracle.py): the edges of the rule that chooses it (2^9 and 2^11 summed
+indices, 2^11 and 2^16 outputs), one and several row groups and workgroups, free axes of
+both sides in any order in C."""
+import numpy as np
+import pytest
+
+import qtorch_amd as qa
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = qa.Context(0)
+    yield c
+    c.close()
+
+
+def _tensordot(a, ra, b, rb, free, pairs, d):
+    """C's flat values; axis i of a tensor is numpy axis -1 - i."""
+    a, b = a.astype(np.complex128).reshape([1 << d] * ra), b.astype(np.complex128).reshape([1 << d] * rb)
+    c = np.tensordot(a, b, axes=([ra - 1 - x for x, _ in pairs], [rb - 1 - y for _, y in pairs]))
+    left = [(True, i) for i in reversed(range(ra)) if i not in [x for x, _ in pairs]]
+    left += [(False, i) for i in reversed(range(rb)) if i not in [y for _, y in pairs]]
+    return c.transpose([left.index(f) for f in reversed(free)]).reshape(-1)
+
+
+# (free wires of A, free wires of B, summed wires, dim_log2)
+SHAPES = [(0, 0, 9, 1), (0, 3, 10, 1), (11, 0, 9, 1), (5, 6, 9, 1), (2, 3, 5, 2), (0, 1, 13, 1), (3, 2, 14, 1),
+          (12, 0, 11, 1), (1, 11, 11, 1), (10, 6, 11, 1), (0, 8, 6, 2), (4, 3, 12, 1)]
+
+
+@pytest.mark.parametrize("prec,tol", [(qa.QT_PLAIN_C128, 0.0), (qa.QT_C64_4M, 2e-6), (qa.QT_C64_3M, 4e-6),
+                                      (qa.QT_C64_BF16X3, 1e-4)])
+@pytest.mark.parametrize("fa,fb,k,d", SHAPES)
+def test_long_sums(ctx, fa, fb, k, d, prec, tol):
+    rng = np.random.default_rng(1000 * fa + 100 * fb + 10 * k + d)
+    c128 = prec == qa.QT_PLAIN_C128
+    dt = np.complex128 if c128 else np.complex64
+    ra, rb = fa + k, fb + k
+    a, b = ((rng.standard_normal(1 << (d * r)) + 1j * rng.standard_normal(1 << (d * r))).astype(dt) for r in (ra, rb))
+    ta, tb = (qa.Tensor(ctx, r, d, qa.QT_DTYPE_C128 if c128 else qa.QT_DTYPE_C64).upload(x)
+              for r, x in ((ra, a), (rb, b)))
+    for interleave in (False, True):
+        pa, pb = rng.permutation(ra), rng.permutation(rb)
+        pairs = [(int(x), int(y)) for x, y in zip(pa[:k], pb[:k])]
+        free = [(True, int(x)) for x in pa[k:]] + [(False, int(y)) for y in pb[k:]]
+        if interleave:
+            free = [free[i] for i in rng.permutation(len(free))]
+        got = qa.contract_pair(ctx, ta, tb, pairs, free, prec)[0].download()
+        ref = _tensordot(a, ra, b, rb, free, pairs, d)
+        # sums of 2^(d k) products of unit variance: rounding of about sqrt(2^(d k)) terms
+        bound = 1e-13 if c128 else tol
+        assert np.abs(got - ref).max() <= bound * np.sqrt(1 << (d * k)) * max(np.abs(ref).max(), 1.0)
