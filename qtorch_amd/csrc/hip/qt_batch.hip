@@ -19,6 +19,7 @@
 #include <cstring>
 #include <map>
 #include <numeric>
+#include <type_traits>
 #include <vector>
 
 #include "qt_batch_impl.h"
@@ -103,7 +104,7 @@ __device__ __forceinline__ void exec_sync() {
 template <class V, int MODE, int LANES, class PA, class PB>
 __device__ __forceinline__ void run_step(PA A, PB B, V* C, const uint32_t* __restrict__ fc,
                                          const uint32_t* __restrict__ gs, int nC, int K, int lane,
-                                         double2* out_final) {
+                                         double2* out_final, V* stage = nullptr) {
     auto put = [&](int c, const Acc<V, MODE>& acc) {
         const V v = acc.get();
         if (out_final) *out_final = double2{double(v.x), double(v.y)};
@@ -156,6 +157,33 @@ __device__ __forceinline__ void run_step(PA A, PB B, V* C, const uint32_t* __res
         if (c < nC) one(c, f0);
         return;
     }
+    if (stage && nC == 1 && K >= 64) {
+        // a long sum into one output (the last step of a network) is one chain of
+        // multiply-adds: a wave loads 64 operand pairs ahead and the chain reads them from
+        // LDS (2^12 complex128 pairs: 430 us with the chain's own loads 4 at a time)
+        if (lane < 64) {
+            const auto pa = A + int(fc[0] & 0xffffu);
+            const auto pb = B + int(fc[0] >> 16);
+            Acc<V, MODE> acc;
+            uint32_t g = gs[lane];
+            V x = pa[int(g & 0xffffu)], y = pb[int(g >> 16)];
+            for (int s = 0; s < K; s += 64) {
+                stage[lane] = x;
+                stage[64 + lane] = y;
+                if (s + 64 < K) {
+                    g = gs[s + 64 + lane];
+                    x = pa[int(g & 0xffffu)];
+                    y = pb[int(g >> 16)];
+                }
+                exec_sync<64, false>();  // the stage is written
+#pragma unroll 16
+                for (int t = 0; t < 64; ++t) acc.mac(stage[t], stage[64 + t]);
+                exec_sync<64, false>();  // and read
+            }
+            if (lane == 0) put(0, acc);
+        }
+        return;
+    }
     uint32_t f_next = lane < nC ? fc[lane] : 0u;
     for (int c = lane; c < nC; c += LANES) {
         const uint32_t f = f_next;
@@ -163,7 +191,20 @@ __device__ __forceinline__ void run_step(PA A, PB B, V* C, const uint32_t* __res
         const auto pa = A + int(f & 0xffffu);
         const auto pb = B + int(f >> 16);
         Acc<V, MODE> acc;
-        if ((K & 3) == 0) {
+        if ((K & 15) == 0) {
+            // 16 operand pairs in flight
+            for (int s = 0; s < K; s += 16) {
+                V x[16], y[16];
+#pragma unroll
+                for (int t = 0; t < 16; ++t) {
+                    const uint32_t g = gs[s + t];
+                    x[t] = pa[int(g & 0xffffu)];
+                    y[t] = pb[int(g >> 16)];
+                }
+#pragma unroll
+                for (int t = 0; t < 16; ++t) acc.mac(x[t], y[t]);
+            }
+        } else if ((K & 3) == 0) {
             // summed extents are powers of D: four independent operand loads in flight
             for (int s = 0; s < K; s += 4) {
                 const uint32_t g0 = gs[s], g1 = gs[s + 1], g2 = gs[s + 2], g3 = gs[s + 3];
@@ -186,6 +227,182 @@ __device__ __forceinline__ void run_step(PA A, PB B, V* C, const uint32_t* __res
     }
 }
 
+// GEMM-shaped steps (C's low bits from A, its high bits from B, 16 or more elements on
+// each side) on the matrix cores, one wavefront per block of BM x BN tiles of 16 x 16
+// outputs.  An MFMA over four k adds its products to the accumulator one at a time, in
+// k's order, each with one rounding (checked on the device: 12,800 of 12,800 results in
+// FP64 and in FP32 equal that chain of FMAs, every other order fails), so k = (s, part)
+// pairs, part 0 then 1, give run_step's chain for every output: re += ax bx, re += -ay by;
+// im += ax by, im += ay bx.  3M's three sums take four s each.  Bit-identical to run_step.
+// Bound by the operand gathers (8 to 16 scattered bytes a lane): the next k-group's are in
+// flight while a k-group's products run.  256 networks of 8.2 million complex128 MACs: 4,957
+// us on the vector steps, 900 us (18.6 of 78.6 TFLOP/s; a step of 256 x 256 outputs over
+// 64 runs at 0.43 of a CU's rate).
+typedef double d4_t __attribute__((ext_vector_type(4)));
+typedef float f4_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ d4_t mfma4(double b, double a, d4_t c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(b, a, c, 0, 0, 0);
+}
+__device__ __forceinline__ f4_t mfma4(float b, float a, f4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(b, a, c, 0, 0, 0);
+}
+
+template <class V, int MODE, int BM, int BN, int UP, class PA, class PB>
+__device__ __forceinline__ void run_step_mfma(PA A, PB B, V* C, const uint32_t* __restrict__ fc,
+                                              const uint32_t* __restrict__ gs, int mb, int nb, int K, int lane,
+                                              int wave, int n_waves) {
+    using T = typename Real<V>::T;
+    using T4 = typename std::conditional<sizeof(T) == 8, d4_t, f4_t>::type;
+    constexpr bool k3M = MODE == QT_C64_3M;
+    constexpr int NA = k3M ? 3 : 2;
+    constexpr int SP = k3M ? 4 : 2;  // s per MFMA
+    const int li = lane & 15, lk = lane >> 4;
+    const int part = lk & 1, ls = k3M ? lk : lk >> 1;
+    const int bmb = mb - 4 - (BM - 1), blocks = 1 << (bmb + nb - 4 - (BN - 1));
+    for (int blk = wave; blk < blocks; blk += n_waves) {
+        const int m0 = (blk & ((1 << bmb) - 1)) * (16 * BM), n0 = (blk >> bmb) * (16 * BN);
+        int oa[BM], ob[BN];
+#pragma unroll
+        for (int i = 0; i < BM; ++i) oa[i] = int(fc[m0 + 16 * i + li] & 0xffffu);
+#pragma unroll
+        for (int j = 0; j < BN; ++j) ob[j] = int(fc[(n0 + 16 * j + li) << mb] >> 16);
+        T4 acc[NA][BN][BM];
+#pragma unroll
+        for (int q = 0; q < NA; ++q)
+#pragma unroll
+            for (int j = 0; j < BN; ++j)
+#pragma unroll
+                for (int i = 0; i < BM; ++i) acc[q][j][i] = T4{0, 0, 0, 0};
+        // 4M and complex128: a lane's A operand is one part of its element
+        T ax[UP][BM], ay[UP][BM], bx[UP][BN], by[UP][BN];
+        uint32_t g[UP];
+        auto offsets = [&](int s0) {
+#pragma unroll
+            for (int u = 0; u < UP; ++u) g[u] = gs[s0 + SP * u + ls];
+        };
+        auto load = [&](T (&x)[UP][BM], T (&y)[UP][BM], T (&z)[UP][BN], T (&w)[UP][BN]) {
+#pragma unroll
+            for (int u = 0; u < UP; ++u) {
+#pragma unroll
+                for (int i = 0; i < BM; ++i) {
+                    const auto p = A + (oa[i] + int(g[u] & 0xffffu));
+                    if constexpr (k3M) {
+                        x[u][i] = p->x;
+                        y[u][i] = p->y;
+                    } else {
+                        x[u][i] = y[u][i] = reinterpret_cast<const T*>(p)[part];
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < BN; ++j) {
+                    const auto p = B + (ob[j] + int(g[u] >> 16));
+                    z[u][j] = p->x;
+                    w[u][j] = p->y;
+                }
+            }
+        };
+        constexpr int kStep = SP * UP;
+        offsets(0);
+        load(ax, ay, bx, by);
+        if (kStep < K) offsets(kStep);
+        for (int s0 = 0; s0 < K; s0 += kStep) {
+            T nax[UP][BM], nay[UP][BM], nbx[UP][BN], nby[UP][BN];
+            if (s0 + kStep < K) {
+                load(nax, nay, nbx, nby);
+                if (s0 + 2 * kStep < K) offsets(s0 + 2 * kStep);
+            }
+#pragma unroll
+            for (int u = 0; u < UP; ++u) {
+                T b0[BN], b1[BN];
+#pragma unroll
+                for (int j = 0; j < BN; ++j) {
+                    const T x = bx[u][j], y = by[u][j];
+                    b0[j] = k3M ? x : part ? -y : x;
+                    b1[j] = k3M ? y : part ? x : y;
+                }
+#pragma unroll
+                for (int j = 0; j < BN; ++j)
+#pragma unroll
+                    for (int i = 0; i < BM; ++i) {
+                        acc[0][j][i] = mfma4(b0[j], ax[u][i], acc[0][j][i]);
+                        acc[1][j][i] = mfma4(b1[j], ay[u][i], acc[1][j][i]);
+                        if constexpr (k3M)
+                            acc[2][j][i] = mfma4(b0[j] + b1[j], ax[u][i] + ay[u][i], acc[2][j][i]);
+                    }
+            }
+            if (s0 + kStep < K) {
+#pragma unroll
+                for (int u = 0; u < UP; ++u) {
+#pragma unroll
+                    for (int i = 0; i < BM; ++i) {
+                        ax[u][i] = nax[u][i];
+                        ay[u][i] = nay[u][i];
+                    }
+#pragma unroll
+                    for (int j = 0; j < BN; ++j) {
+                        bx[u][j] = nbx[u][j];
+                        by[u][j] = nby[u][j];
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < BN; ++j)
+#pragma unroll
+            for (int i = 0; i < BM; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    // item r of a lane: row (n) lk + 4 r in FP64, 4 lk + r in FP32; column (m) li
+                    const int n = n0 + 16 * j + (sizeof(T) == 8 ? lk + 4 * r : 4 * lk + r);
+                    V v;
+                    if constexpr (k3M) {
+                        v.x = acc[0][j][i][r] - acc[1][j][i][r];
+                        v.y = acc[2][j][i][r] - acc[0][j][i][r] - acc[1][j][i][r];
+                    } else {
+                        v.x = acc[0][j][i][r];
+                        v.y = acc[1][j][i][r];
+                    }
+                    C[(m0 + 16 * i + li) + (n << mb)] = v;
+                }
+    }
+}
+
+// Steps of at least 2^12 MACs with 16 or more elements on each side and 4 or more summed
+// indices: below that a wave's lanes finish the step sooner one output each (a 16 x 16
+// output over four summed indices is one tile, which leaves three of four waves idle).
+constexpr int32_t kStepMfma = 2;
+inline int32_t mfma_flags(int mbits, int nbits, int k_bits) {
+    const bool ok = mbits >= 4 && nbits >= 4 && k_bits >= 2 && mbits + nbits + k_bits >= 12;
+    return ok ? kStepMfma | (mbits << 8) : 0;
+}
+
+template <class V, int MODE, int LANES, class PA, class PB>
+__device__ __forceinline__ void run_step_any(PA A, PB B, V* C, const uint32_t* __restrict__ fc,
+                                             const uint32_t* __restrict__ gs, const StepDesc& st, int lane,
+                                             double2* out_final, V* stage) {
+    if constexpr (LANES >= 64 && MODE != QT_C64_BF16X3) {
+        if (st.flags & kStepMfma) {
+            const int mb = (st.flags >> 8) & 0xff, nb = st.nc_bits - mb, K = 1 << st.k_bits;
+            constexpr int kWaves = LANES / 64;
+            const int l = lane & 63, w = lane >> 6;
+            // k-groups of 4 s in complex128 and in narrow blocks (registers), else of 8
+            constexpr int U4 = MODE == QT_C64_3M ? 1 : 2, U8 = sizeof(V) == 16 ? U4 : 2 * U4;
+            const int blocks = mb + nb - 8;  // log2 of the 16 x 16 tiles: blocks of 2 x 2 when every wave gets one
+            if (K >= 8 && blocks >= 4 && mb >= 5 && nb >= 5)
+                run_step_mfma<V, MODE, 2, 2, U8>(A, B, C, fc, gs, mb, nb, K, l, w, kWaves);
+            else if (K >= 8 && blocks >= 3 && nb >= 5)
+                run_step_mfma<V, MODE, 1, 2, U8>(A, B, C, fc, gs, mb, nb, K, l, w, kWaves);
+            else if (K >= 8 && blocks >= 3)
+                run_step_mfma<V, MODE, 2, 1, U8>(A, B, C, fc, gs, mb, nb, K, l, w, kWaves);
+            else
+                run_step_mfma<V, MODE, 1, 1, U4>(A, B, C, fc, gs, mb, nb, K, l, w, kWaves);
+            return;
+        }
+    }
+    run_step<V, MODE, LANES>(A, B, C, fc, gs, 1 << st.nc_bits, 1 << st.k_bits, lane, out_final, stage);
+}
+
 // With TOUT, every instance's last step writes its whole result (a tensor, or a
 // scalar) to the instance's output tensor tout[i] instead of the FP64 value array.
 template <class V, int MODE, int LANES, bool GLOBAL_SCRATCH, bool TOUT>
@@ -193,18 +410,21 @@ __global__ __launch_bounds__(kWg) void k_batch(const ProgHdr* __restrict__ progs
                                                const uint32_t* __restrict__ tabs,
                                                const int64_t* __restrict__ leaf_refs, const V* __restrict__ pool,
                                                const Instance* __restrict__ inst, int n_inst,
-                                               int32_t* __restrict__ counter, double2* __restrict__ out,
-                                               V* __restrict__ gscratch, int scratch_elems,
-                                               V* const* __restrict__ tout) {
+                                               const int32_t* __restrict__ order, int32_t* __restrict__ counter,
+                                               double2* __restrict__ out, V* __restrict__ gscratch,
+                                               int scratch_elems, V* const* __restrict__ tout) {
     extern __shared__ unsigned char lds_raw[];
     __shared__ int wg_next;
     constexpr int kExec = kWg / LANES;
     const int ex = threadIdx.x / LANES;
     const int lane = threadIdx.x % LANES;
     V* mem;
-    if constexpr (GLOBAL_SCRATCH)
+    V* stage = nullptr;  // of the executor's (first) wave, where intermediates are in device memory
+    if constexpr (GLOBAL_SCRATCH) {
+        __shared__ V stages[kExec][128];
+        stage = stages[ex];
         mem = gscratch + (int64_t(blockIdx.x) * kExec + ex) * scratch_elems;
-    else
+    } else
         mem = reinterpret_cast<V*>(lds_raw) + ex * scratch_elems;
     while (true) {
         int i;
@@ -220,14 +440,16 @@ __global__ __launch_bounds__(kWg) void k_batch(const ProgHdr* __restrict__ progs
         }
         i = __builtin_amdgcn_readfirstlane(i);
         if (i >= n_inst) break;
+        if (order) i = __builtin_amdgcn_readfirstlane(order[i]);
         const Instance in = inst[i];
         const ProgHdr P = progs[in.prog];
         const int64_t* refs = leaf_refs + P.leaf_begin;
+        StepDesc next = steps[P.step_begin];
         for (int si = 0; si < P.n_steps; ++si) {
-            const StepDesc st = steps[P.step_begin + si];
+            const StepDesc st = next;
+            if (si + 1 < P.n_steps) next = steps[P.step_begin + si + 1];  // in flight during this step
             const uint32_t* fc = tabs + st.tab;
-            const int nC = 1 << st.nc_bits, K = 1 << st.k_bits;
-            const uint32_t* gs = fc + nC;
+            const uint32_t* gs = fc + (1 << st.nc_bits);
             double2* fin = (st.flags & 1) ? out + i : nullptr;
             V* C = mem + st.c;
             if constexpr (TOUT) {
@@ -243,14 +465,13 @@ __global__ __launch_bounds__(kWg) void k_batch(const ProgHdr* __restrict__ progs
                 return pool + off;
             };
             if (st.a < 0 && st.b < 0)
-                run_step<V, MODE, LANES>(leaf(st.a), leaf(st.b), C, fc, gs, nC, K, lane, fin);
+                run_step_any<V, MODE, LANES>(leaf(st.a), leaf(st.b), C, fc, gs, st, lane, fin, stage);
             else if (st.a < 0)
-                run_step<V, MODE, LANES>(leaf(st.a), (const V*)(mem + st.b), C, fc, gs, nC, K, lane, fin);
+                run_step_any<V, MODE, LANES>(leaf(st.a), (const V*)(mem + st.b), C, fc, gs, st, lane, fin, stage);
             else if (st.b < 0)
-                run_step<V, MODE, LANES>((const V*)(mem + st.a), leaf(st.b), C, fc, gs, nC, K, lane, fin);
+                run_step_any<V, MODE, LANES>((const V*)(mem + st.a), leaf(st.b), C, fc, gs, st, lane, fin, stage);
             else
-                run_step<V, MODE, LANES>((const V*)(mem + st.a), (const V*)(mem + st.b), C, fc, gs, nC, K, lane,
-                                         fin);
+                run_step_any<V, MODE, LANES>((const V*)(mem + st.a), (const V*)(mem + st.b), C, fc, gs, st, lane, fin, stage);
             exec_sync<LANES, GLOBAL_SCRATCH>();
         }
     }
@@ -383,11 +604,6 @@ __global__ void k_group_sum(const double2* __restrict__ out, const int32_t* __re
     if (threadIdx.x == 0) sums[g] = acc;
 }
 
-__global__ void k_to_c64(const double2* __restrict__ in, float2* __restrict__ out, int64_t n) {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = float2{float(in[i].x), float(in[i].y)};
-}
-
 // Device array of at least n elements, reused while it is large enough (contents
 // not kept), then filled from src if src is given.
 template <class T>
@@ -424,7 +640,13 @@ inline size_t grouped_lds_elems(const qt_batch* b) {
     return (b->use_global_scratch ? 0 : w * size_t(b->slot_stride)) +
            (b->stage_leaves ? w * size_t(b->pstage) + size_t(b->cstage) : 0);
 }
-inline int grid_wgs(const qt_batch* b) { return b->n_cus * b->wgs_per_cu * (b->lanes >= 64 ? 1 : 4); }
+inline int grid_wgs(const qt_batch* b) {
+    if (b->lanes < 64) return b->n_cus * b->wgs_per_cu * 4;
+    // no more workgroups than the instances need, so that one goes to every CU before
+    // any CU gets two
+    const int per = execs_per_wg(b->lanes);
+    return std::min(b->n_cus * b->wgs_per_cu, std::max(b->n_cus, (b->n_inst + per - 1) / per));
+}
 
 template <class V, int MODE>
 qt_status launch_grouped_t(qt_batch* b) {
@@ -471,7 +693,7 @@ qt_status launch_batch_t(qt_batch* b) {
     }
     Ctx* c = b->ctx;
     const int kExec = kWg / b->lanes;
-    const unsigned grid = unsigned(b->n_cus * b->wgs_per_cu);
+    const unsigned grid = unsigned(grid_wgs(b));
     const size_t lds = b->use_global_scratch ? 0 : size_t(kExec) * size_t(b->scratch_elems) * sizeof(V);
     V* gs = static_cast<V*>(b->d_global_scratch);
     const V* pool = static_cast<const V*>(b->d_pool);
@@ -479,8 +701,8 @@ qt_status launch_batch_t(qt_batch* b) {
     V* const* tout = reinterpret_cast<V* const*>(b->d_tout);
 #define QT_LAUNCH_T(L, G, T)                                                                                       \
     hipLaunchKernelGGL((k_batch<V, MODE, L, G, T>), dim3(grid), dim3(kWg), lds, c->stream, b->d_progs, b->d_steps, \
-                       b->d_tabs, b->d_leaf_refs, pool, b->d_inst, b->n_inst, b->d_counter, d_out, gs,            \
-                       b->scratch_elems, tout)
+                       b->d_tabs, b->d_leaf_refs, pool, b->d_inst, b->n_inst, b->d_order, b->d_counter, d_out,    \
+                       gs, b->scratch_elems, tout)
 #define QT_LAUNCH(L, G)              \
     if (b->tensor_out) {             \
         QT_LAUNCH_T(L, G, true);     \
@@ -545,6 +767,30 @@ qt_status launch_batch(qt_batch* b, bool capture = false) {
 
 size_t elem_size(int precision) { return precision == QT_PLAIN_C128 ? 16 : 8; }
 
+// The order in which executors of 64 or more lanes take the instances: the longest
+// programs first, so that none of them starts while the others run out.  Uniform batches
+// (within a factor of two) keep the instances' own order.
+qt_status order_instances(qt_batch* b) {
+    int64_t least = INT64_MAX, most = 0;
+    for (int i = 0; i < b->n_inst; ++i) {
+        const int64_t m = b->prog_cmacs[size_t(b->h_prog[size_t(i)])];
+        least = std::min(least, m);
+        most = std::max(most, m);
+    }
+    const bool on = b->n_inst > 1 && most / 2 > least;
+    std::vector<int32_t> order;
+    if (on) {
+        order.resize(size_t(b->n_inst));
+        std::iota(order.begin(), order.end(), 0);
+        std::stable_sort(order.begin(), order.end(), [&](int32_t x, int32_t y) {
+            return b->prog_cmacs[size_t(b->h_prog[size_t(x)])] > b->prog_cmacs[size_t(b->h_prog[size_t(y)])];
+        });
+    }
+    qt_status s = dev_put(b->ctx, &b->d_order_mem, &b->cap_order, order.data(), order.size());
+    b->d_order = on && s == QT_OK ? b->d_order_mem : nullptr;
+    return s;
+}
+
 qt_status configure_scratch(qt_batch* b) {
     Ctx* c = b->ctx;
     b->shape_ok = false;  // set once the arrays below match the executor shape
@@ -581,6 +827,10 @@ qt_status configure_scratch(qt_batch* b) {
         qt_status s = dev_put(c, &b->d_chunks, &b->cap_chunks, ch.data(), ch.size());
         if (s != QT_OK) return s;
         b->n_chunks = int(ch.size());
+    }
+    else {
+        qt_status s = order_instances(b);
+        if (s != QT_OK) return s;
     }
     if (b->use_global_scratch) {
         const size_t need = size_t(grid_wgs(b)) * size_t(kExec) * size_t(b->slot_stride) * es;
@@ -993,7 +1243,11 @@ qt_status qt_program_create(qt_ctx* cx, int dim_log2, int n_leaves, const int32_
         st.a = a < n_leaves ? -(1 + a) : slot[size_t(a - n_leaves)];
         st.b = b < n_leaves ? -(1 + b) : slot[size_t(b - n_leaves)];
         st.c = s + 1 < n_steps ? slot[size_t(s)] : 0;
-        st.flags = s + 1 == n_steps ? 1 : 0;
+        int mbits = 0;  // C's low bits from A, its high bits from B (src/Network.h:739-769)?
+        while (mbits < st.nc_bits && c_src[size_t(mbits)] < 64) ++mbits;
+        bool split = true;
+        for (int i = mbits; i < st.nc_bits; ++i) split = split && c_src[size_t(i)] >= 64;
+        st.flags = (s + 1 == n_steps ? 1 : 0) | (split ? qt::mfma_flags(mbits, st.nc_bits - mbits, st.k_bits) : 0);
         st.pad = (ra * dl) | ((rb * dl) << 8);  // element bits of the operands (leaf staging)
         p->steps.push_back(st);
         p->cmacs += int64_t(1) << ((rc + k) * dl);
@@ -1044,7 +1298,14 @@ qt_status qt_batch_create(qt_ctx* cx, int n_programs, qt_program* const* progs, 
         // default executor shape from the scratch footprint (the autotuner may refine it)
         const size_t per_exec = size_t(b->scratch_elems) * qt::elem_size(precision);
         b->lanes = per_exec * 4 <= 16 * 1024 ? 64 : 256;
-        b->wgs_per_cu = per_exec * 4 <= 16 * 1024 ? 4 : per_exec <= 32 * 1024 ? 2 : 1;
+        // workgroup executors wait on memory most of the time, four to a CU hide some of
+        // it: 1,920 complex64 networks of 0.01 to 10 million MACs, intermediates in device
+        // memory, take 1,465 / 928 / 843 us at 1 / 2 / 4 (two where that keeps the
+        // intermediates in LDS; fewer where the scratch area would pass 4 GiB)
+        b->wgs_per_cu = per_exec > 32 * 1024 && per_exec <= 64 * 1024 ? 2 : 4;
+        while (b->lanes == 256 && b->wgs_per_cu > 1 &&
+               per_exec * size_t(b->n_cus) * size_t(b->wgs_per_cu) > (size_t(4) << 30))
+            b->wgs_per_cu /= 2;
         s = qt::configure_scratch(b.get());
     }
     if (s != QT_OK) {
@@ -1475,7 +1736,7 @@ qt_status qt_batch_destroy(qt_batch* b) {
                         (void*)b->d_inst, (void*)b->d_out, (void*)b->d_counter, (void*)b->d_seg, (void*)b->d_members,
                         (void*)b->d_group, b->d_global_scratch, (void*)b->d_chunks, b->d_pool_stage,
                         (void*)b->d_leaf_lds, (void*)b->d_csts, (void*)b->d_tout, (void*)b->d_schunks,
-                        (void*)b->d_out_prev, (void*)b->d_param_status, (void*)b->d_angles, b->d_rot_desc})
+                        (void*)b->d_out_prev, (void*)b->d_order_mem, (void*)b->d_param_status, (void*)b->d_angles, b->d_rot_desc})
             qt::batch_free(b->ctx, p);
         --b->ctx->live;
     }

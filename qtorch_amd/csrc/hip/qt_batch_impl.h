@@ -47,7 +47,7 @@ struct StepDesc {
     int32_t tab;        // offset of the step's tables in the table array (uint32 units)
     int32_t nc_bits;    // output elements = 1 << nc_bits
     int32_t k_bits;     // summed elements = 1 << k_bits
-    int32_t flags;      // bit 0: final step
+    int32_t flags;      // bit 0: final step; bit 1: runs on the matrix cores, A's output bits in bits 8-15
     int32_t pad;
 };
 
@@ -92,6 +92,9 @@ struct qt_batch {
     double* d_out = nullptr;       // 2 * n_inst
     size_t cap_inst = 0, cap_out = 0, cap_seg = 0, cap_members = 0, cap_group = 0, cap_chunks = 0;
     int32_t* d_counter = nullptr;
+    int32_t* d_order_mem = nullptr;      // instances, longest program first
+    const int32_t* d_order = nullptr;    // d_order_mem, or null: the instances' own order
+    size_t cap_order = 0;
     // group sums
     int32_t* d_seg = nullptr;
     int32_t* d_members = nullptr;

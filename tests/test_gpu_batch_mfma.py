@@ -1,0 +1,55 @@
+"""Program steps on the matrix cores (executors of 64 and 256 lanes) against the vector
+steps of lane groups: the same chain of multiply-adds per output, so the same bits."""
+import math
+import os
+
+import numpy as np
+import pytest
+
+import qtorch_amd as qa
+from qtorch_amd import workloads as wl
+
+GOLDEN_DIR = os.path.join(os.path.dirname(__file__), "golden")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = qa.Context(0)
+    yield c
+    c.close()
+
+
+def _same_bits(batch):
+    batch.config(16, 1, qa.QT_SCRATCH_GLOBAL)
+    batch.launch()
+    ref = batch.results()
+    for lanes, wgs in ((64, 1), (256, 1), (256, 4)):
+        batch.config(lanes, wgs, qa.QT_SCRATCH_GLOBAL)
+        batch.launch()
+        got = batch.results()
+        for x, y in zip(ref, got):
+            assert np.array_equal(x, y), (lanes, wgs)
+
+
+@pytest.mark.parametrize("prec", [qa.QT_PLAIN_C128, qa.QT_C64_4M, qa.QT_C64_3M])
+def test_light_cones_of_uneven_size(ctx, prec):
+    """Depth 2 on a 3-regular graph: programs of uneven size, taken longest first."""
+    rng = np.random.default_rng(3)
+    with open(os.path.join(GOLDEN_DIR, "samples", "3regRand30Node50.dgf")) as f:
+        b = qa.QaoaBatch(ctx, f.read(), 2, ref_map=False, precision=prec)
+    b.set_angles(np.concatenate([rng.uniform(0, math.pi / 2, (3, 2)), rng.uniform(-3, 3, (3, 2))], axis=1))
+    _same_bits(b)
+    b.close()
+
+
+@pytest.mark.parametrize("prec", [qa.QT_PLAIN_C128, qa.QT_C64_4M, qa.QT_C64_3M])
+@pytest.mark.parametrize("dim_log2,rows,cols,depth", [(1, 3, 4, 8), (2, 2, 3, 6)])
+def test_grid_networks(ctx, prec, dim_log2, rows, cols, depth):
+    """Dimension 2 (any power of two summed, 8 included) and 4."""
+    q = wl.grid_random_circuit(rows, cols, depth, seed=5)
+    n = rows * cols
+    b = qa.NetBatch(ctx, [q] * 5, [wl.measure_text(wl.bitstring(n, k)) for k in range(5)], precision=prec,
+                    dim_log2=dim_log2)
+    _same_bits(b)
+    b.close()
