@@ -597,6 +597,19 @@ __global__ __launch_bounds__(kThreads) void k_permute(const V* __restrict__ in, 
     }
 }
 
+// Output tile of a workgroup (tile counts are powers of two).  Workgroups go to the eight
+// XCDs in turn, each with its own L2: XCD x takes the x-th eighth of the tiles, in columns
+// of up to 8 tiles of m, so that the 32 to 64 tiles it runs at once share 8 panels of A'
+// and 4 to 8 of B' instead of one of B' and as many of A' as there are tiles.
+__device__ __forceinline__ void gemm_tile(int64_t id, int64_t tiles_m, int64_t tiles_n, int64_t& tm, int64_t& tn) {
+    const int64_t total = tiles_m * tiles_n;
+    if (total >= 64) id = (id & 7) * (total >> 3) + (id >> 3);
+    const int64_t gm = tiles_m < 8 ? tiles_m : 8;
+    const int64_t per = gm * tiles_n, g = id / per, r = id % per;
+    tm = g * gm + r % gm;
+    tn = r / gm;
+}
+
 // Complex FP64 GEMM on MFMA: C[m + M n] = sum_s A'[s][m] * B'[s][n].
 // 64x64 output tile per workgroup, four waves of 32x32; each 16x16 block of a wave
 // takes four real v_mfma_f64_16x16x4f64 per k-step of 4 (re*re, -im*im, re*im, im*re).
@@ -604,13 +617,13 @@ __global__ __launch_bounds__(kThreads) void k_permute(const V* __restrict__ in, 
 // the lanes of one accumulator row hold 16 consecutive m and store contiguously.
 constexpr int GM = 64, GN = 64, GK = 16;
 typedef double d4_t __attribute__((ext_vector_type(4)));
+typedef double d2_t __attribute__((ext_vector_type(2)));
 
-__global__ __launch_bounds__(kThreads) void k_gemm_c128(const double2* __restrict__ Ap,
+__global__ __launch_bounds__(kThreads, 2) void k_gemm_c128(const double2* __restrict__ Ap,
                                                         const double2* __restrict__ Bp,
                                                         double2* __restrict__ C, int64_t M,
                                                         int64_t N, int64_t K) {
-    __shared__ double as_re[GK][GM + 1], as_im[GK][GM + 1];
-    __shared__ double bs_re[GK][GN + 1], bs_im[GK][GN + 1];
+    __shared__ d2_t sa[2][GK][GM], sb[2][GK][GN];  // two k-tiles: one barrier per k-tile
     // split K: workgroups with blockIdx.z = z take summed rows [z K, (z + 1) K) and write
     // their own M x N partial product at C + z M N
     Ap += int64_t(blockIdx.z) * K * M;
@@ -621,7 +634,9 @@ __global__ __launch_bounds__(kThreads) void k_gemm_c128(const double2* __restric
     const int64_t tiles_m = M / GM;
     const int64_t tile = int64_t(blockIdx.x) + int64_t(blockIdx.y) * gridDim.x;
     if (tile >= tiles_m * (N / GN)) return;
-    const int64_t m0 = (tile % tiles_m) * GM, n0 = (tile / tiles_m) * GN;
+    int64_t tm, tn;
+    gemm_tile(tile, tiles_m, N / GN, tm, tn);
+    const int64_t m0 = tm * GM, n0 = tn * GN;
     d4_t acc_re[2][2], acc_im[2][2];
     for (int i = 0; i < 2; ++i)
         for (int j = 0; j < 2; ++j) {
@@ -629,49 +644,54 @@ __global__ __launch_bounds__(kThreads) void k_gemm_c128(const double2* __restric
             acc_im[i][j] = d4_t{0, 0, 0, 0};
         }
     const int li = lane & 15, lk = lane >> 4;
-    // each thread stages kPer elements of A' and of B' per k-tile; the next k-tile is
-    // loaded into registers while the current one is multiplied from LDS.  A last
+    // each thread stages kPer elements of A' and of B' per k-tile: rows (tid / 64) + 4 q; the
+    // next k-tile is in flight while the current one is multiplied from LDS.  A last
     // k-tile beyond K (K = 8) is filled with zeros, which add nothing.
     constexpr int kPer = GK * GM / kThreads;
-    static_assert(GK * GM == GK * GN && kPer * kThreads == GK * GM, "tile staging");
-    double2 ra[kPer], rb[kPer];
+    static_assert(GM == 64 && GN == 64 && kPer * kThreads == GK * GM, "tile staging");
+    d2_t ra[kPer], rb[kPer];
+    const d2_t* pa = reinterpret_cast<const d2_t*>(Ap) + int64_t(wave) * M + m0 + lane;
+    const d2_t* pb = reinterpret_cast<const d2_t*>(Bp) + int64_t(wave) * N + n0 + lane;
     auto fetch = [&](int64_t k0) {
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
-            const int e = tid + q * kThreads, kk = e / GM, rr = e % GM;
-            const bool in_k = k0 + kk < K;
-            ra[q] = in_k ? Ap[(k0 + kk) * M + m0 + rr] : double2{0.0, 0.0};
-            rb[q] = in_k ? Bp[(k0 + kk) * N + n0 + rr] : double2{0.0, 0.0};
+            const bool in_k = k0 + wave + 4 * q < K;
+            ra[q] = in_k ? pa[4 * q * M] : d2_t{0.0, 0.0};
+            rb[q] = in_k ? pb[4 * q * N] : d2_t{0.0, 0.0};
+        }
+        pa += GK * M;
+        pb += GK * N;
+    };
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+            sa[buf][wave + 4 * q][lane] = ra[q];
+            sb[buf][wave + 4 * q][lane] = rb[q];
         }
     };
     fetch(0);
-    for (int64_t k0 = 0; k0 < K; k0 += GK) {
-#pragma unroll
-        for (int q = 0; q < kPer; ++q) {
-            const int e = tid + q * kThreads, kk = e / GM, rr = e % GM;
-            as_re[kk][rr] = ra[q].x;
-            as_im[kk][rr] = ra[q].y;
-            bs_re[kk][rr] = rb[q].x;
-            bs_im[kk][rr] = rb[q].y;
-        }
-        __syncthreads();
-        if (k0 + GK < K) fetch(k0 + GK);
+    stage(0);
+    __syncthreads();
+    int buf = 0;
+    for (int64_t k0 = 0; k0 < K; k0 += GK, buf ^= 1) {
+        const bool more = k0 + GK < K;
+        if (more) fetch(k0 + GK);
 #pragma unroll
         for (int kk = 0; kk < GK; kk += 4) {
             const int kl = kk + lk;
             double are[2], aim[2];
 #pragma unroll
             for (int bm = 0; bm < 2; ++bm) {
-                const int mm = wm * 32 + bm * 16 + li;
-                are[bm] = as_re[kl][mm];
-                aim[bm] = as_im[kl][mm];
+                const d2_t v = sa[buf][kl][wm * 32 + bm * 16 + li];
+                are[bm] = v.x;
+                aim[bm] = v.y;
             }
             double bre[2], bim[2];
 #pragma unroll
             for (int bn = 0; bn < 2; ++bn) {
-                const int nn = wn * 32 + bn * 16 + li;
-                bre[bn] = bs_re[kl][nn];
-                bim[bn] = bs_im[kl][nn];
+                const d2_t v = sb[buf][kl][wn * 32 + bn * 16 + li];
+                bre[bn] = v.x;
+                bim[bn] = v.y;
             }
             // the four products of a block go to two accumulators; issuing them in
             // four rounds over the blocks keeps dependent MFMAs apart
@@ -696,6 +716,7 @@ __global__ __launch_bounds__(kThreads) void k_gemm_c128(const double2* __restric
                 for (int bm = 0; bm < 2; ++bm)
                     acc_im[bn][bm] = __builtin_amdgcn_mfma_f64_16x16x4f64(bre[bn], aim[bm], acc_im[bn][bm], 0, 0, 0);
         }
+        if (more) stage(buf ^ 1);  // read last in the k-tile before, behind its barrier
         __syncthreads();
     }
 #pragma unroll
@@ -1307,11 +1328,13 @@ __global__ __launch_bounds__(kThreads) void k_sum_splits(const float4* __restric
     C[i] = a;
 }
 
+// Two workgroups a CU (4M: 128 accumulation registers of 256) cover each other's barriers
+// and LDS latency; 3M's 192 leave room for one.
 template <int MODE>
-__global__ __launch_bounds__(kThreads) void k_gemm_c64_big(const float2* __restrict__ Ap,
-                                                           const float2* __restrict__ Bp, float2* __restrict__ C,
-                                                           int64_t M, int64_t N, int64_t K) {
-    __shared__ float sa[2][BK * BROW], sb[2][BK * BROW];  // [re|im][k][row]
+__global__ __launch_bounds__(kThreads, MODE == MODE_3M ? 1 : 2) void k_gemm_c64_big(
+    const float2* __restrict__ Ap, const float2* __restrict__ Bp, float2* __restrict__ C, int64_t M, int64_t N,
+    int64_t K) {
+    __shared__ float2 sa[2][BK * BROW], sb[2][BK * BROW];  // [buffer][k][row]
     // split K: workgroups with blockIdx.z = z take summed rows [z K, (z + 1) K) and write
     // their own M x N partial product at C + z M N
     Ap += int64_t(blockIdx.z) * K * M;
@@ -1323,7 +1346,9 @@ __global__ __launch_bounds__(kThreads) void k_gemm_c64_big(const float2* __restr
     const int64_t tiles_m = M / BT;
     const int64_t tile = int64_t(blockIdx.x) + int64_t(blockIdx.y) * gridDim.x;
     if (tile >= tiles_m * (N / BT)) return;
-    const int64_t m0 = (tile % tiles_m) * BT, n0 = (tile / tiles_m) * BT;
+    int64_t tm, tn;
+    gemm_tile(tile, tiles_m, N / BT, tm, tn);
+    const int64_t m0 = tm * BT, n0 = tn * BT;
     constexpr int NA = MODE == MODE_3M ? 3 : 2;
     f4_t acc[NA][4][4];
 #pragma unroll
@@ -1332,38 +1357,46 @@ __global__ __launch_bounds__(kThreads) void k_gemm_c64_big(const float2* __restr
         for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int j = 0; j < 4; ++j) acc[q][i][j] = f4_t{0, 0, 0, 0};
-    // each thread moves 8 elements of A' and 8 of B' per k-tile: element e = tid + 256 q
-    float2 ra[8], rb[8];
-    auto fetch = [&](int64_t k0) {
+    // each thread moves 8 elements of A' and 8 of B' per k-tile, two neighbours per load:
+    // rows (tid / 64) + 4 q, elements 2 (tid % 64) and the next
+    f4_t ra[4], rb[4];
+    const float2* pa = Ap + int64_t(tid >> 6) * M + m0 + 2 * (tid & 63);
+    const float2* pb = Bp + int64_t(tid >> 6) * N + n0 + 2 * (tid & 63);
+    auto fetch = [&]() {
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const int e = tid + kThreads * q, kk = e / BT, rr = e % BT;
-            ra[q] = Ap[(k0 + kk) * M + m0 + rr];
-            rb[q] = Bp[(k0 + kk) * N + n0 + rr];
+        for (int q = 0; q < 4; ++q) {
+            ra[q] = *reinterpret_cast<const f4_t*>(pa + 4 * q * M);
+            rb[q] = *reinterpret_cast<const f4_t*>(pb + 4 * q * N);
+        }
+        pa += BK * M;
+        pb += BK * N;
+    };
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int o = ((tid >> 6) + 4 * q) * BROW + 2 * (tid & 63);
+            *reinterpret_cast<f4_t*>(&sa[buf][o]) = ra[q];
+            *reinterpret_cast<f4_t*>(&sb[buf][o]) = rb[q];
         }
     };
-    fetch(0);
-    for (int64_t k0 = 0; k0 < K; k0 += BK) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const int e = tid + kThreads * q, o = (e / BT) * BROW + e % BT;
-            sa[0][o] = ra[q].x;
-            sa[1][o] = ra[q].y;
-            sb[0][o] = rb[q].x;
-            sb[1][o] = rb[q].y;
-        }
-        __syncthreads();
-        if (k0 + BK < K) fetch(k0 + BK);
+    fetch();
+    stage(0);
+    __syncthreads();
+    int buf = 0;
+    for (int64_t k0 = 0; k0 < K; k0 += BK, buf ^= 1) {
+        const bool more = k0 + BK < K;
+        if (more) fetch();
 #pragma unroll
         for (int kk = 0; kk < BK; kk += 4) {
             const int o = (kk + lk) * BROW;
             float ar[4], ai[4], br[4], bi[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                ar[i] = sa[0][o + wm * 64 + i * 16 + li];
-                ai[i] = sa[1][o + wm * 64 + i * 16 + li];
-                br[i] = sb[0][o + wn * 64 + i * 16 + li];
-                bi[i] = sb[1][o + wn * 64 + i * 16 + li];
+                const float2 va = sa[buf][o + wm * 64 + i * 16 + li], vb = sb[buf][o + wn * 64 + i * 16 + li];
+                ar[i] = va.x;
+                ai[i] = va.y;
+                br[i] = vb.x;
+                bi[i] = vb.y;
             }
             // one round of MFMAs over all 16 blocks per product, so that no MFMA waits
             // for the one just before it
@@ -1412,6 +1445,7 @@ __global__ __launch_bounds__(kThreads) void k_gemm_c64_big(const float2* __restr
                         acc[1][bn][bm] = __builtin_amdgcn_mfma_f32_16x16x4f32(br[bn], ai[bm], acc[1][bn][bm], 0, 0, 0);
             }
         }
+        if (more) stage(buf ^ 1);  // read last in the k-tile before, behind its barrier
         __syncthreads();
     }
 #pragma unroll
