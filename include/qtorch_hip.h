@@ -143,6 +143,25 @@ qt_status qt_contract_pair_noalloc(qt_ctx* ctx, const qt_tensor* A, int rank_a, 
                                    int rank_c, const int32_t* free_src, qt_tensor* C, int precision,
                                    int64_t* cmacs);
 
+/* Several consecutive pairwise steps on one growing tensor in a single pass over it (the
+ * steps of a circuit sweep: a large tensor and a small one at a time).  Link i contracts
+ * the tensor so far (operand A) with the small tensor G[i] (operand B):
+ *   desc : 3 ints per link: rank of G[i], k, rank of the result
+ *   axes : per link pair_x[k], pair_g[k], free_src[rank of the result], concatenated (the
+ *          conventions of qt_contract_pair)
+ * qt_chain_links returns how many of the n links one pass takes, counted from the first
+ * (0: fewer than two; they go through qt_contract_pair): up to 8 links on a tensor of 2^16
+ * elements or more, each with one or two summed index bits, at most two new ones, and the
+ * tensor's free axes in their order before the small one's.  Host only.
+ * qt_contract_chain runs exactly n such links (QT_UNSUPPORTED if they do not fit a pass, or
+ * if a small tensor carries a power-of-two exponent) into C, a distinct, allocated tensor
+ * of the last link's rank.  Every step has qt_contract_pair's arithmetic and order, so
+ * without QT_RESCALE the result equals the steps one by one bit for bit; with it, C is
+ * scaled once, after the last link.  Asynchronous on the context's stream. */
+int qt_chain_links(int rank_x, int dim_log2, int dtype, int n, const int32_t* desc, const int32_t* axes);
+qt_status qt_contract_chain(qt_ctx* ctx, const qt_tensor* X, int rank_x, int n, const qt_tensor* const* G,
+                            const int32_t* desc, const int32_t* axes, qt_tensor* C, int precision);
+
 /* Reads the rank-0 result of a finished contraction (the mFinalVal read of
  * src/Network.h:961-969 and src/LineGraph.h:388), with a rescaled tensor's exponent
  * applied in FP64; synchronises. */

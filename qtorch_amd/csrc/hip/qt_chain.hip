@@ -1,0 +1,420 @@
+// Chains of thin contraction steps in one pass over the large tensor (libqtorch_hip.so).
+//
+// A circuit sweep contracts one growing tensor with a small tensor at a time: each step
+// sums one or two index bits of it and adds up to two.  Step by step (k_thin) every step
+// reads and writes the whole tensor.  k_chain takes several consecutive steps: a workgroup
+// loads a tile of the tensor into LDS, namely every value of the bits that the steps sum
+// and of the lowest bits (whole cache lines), runs the steps on it there, and writes the
+// result's tile.  Each step does k_thin's arithmetic in its order, so the results have
+// the bits that the steps one by one give.
+#include <algorithm>
+#include <cstring>
+#include <vector>
+
+#include "qt_internal.h"
+#include "qt_mac.h"
+
+namespace qt {
+
+namespace {
+
+constexpr int kMaxLinks = 8;     // steps of one pass
+constexpr int kThreadBits = 8;  // two workgroups a CU (LDS); 512 threads measured 4 %, 1,024 35 % slower
+constexpr int kChainThreads = 1 << kThreadBits;
+constexpr int kMaxTileBits = 12; // complex64; one less in complex128 (two buffers of 32 KB)
+
+struct ChainStep {
+    int32_t ns, nb;       // summed bits (1 or 2) and added bits (0 to 2)
+    int32_t lb;           // tile bits before the step
+    int32_t adj;          // the summed bit at tile position 0, or -1
+    int32_t ins[2];       // tile positions of the summed bits, ascending
+    int32_t off[4];       // tile offset of summed index j
+    int32_t g_small[4];   // small operand offset of summed index j
+    int32_t g_free[4];    // small operand offset of its free part o
+};
+
+// Tile bits are the tensor's bits in increasing position; each step takes its summed bits
+// away and adds the new ones on top, as in the step's result.
+struct ChainPlan {
+    int32_t n_steps, tb_in, tb_out, n_rest;
+    int32_t in_pos[kMaxTileBits], out_pos[kMaxTileBits];
+    int32_t rest_in[48], rest_out[48];
+    ChainStep step[kMaxLinks];
+};
+
+struct ChainArgs {
+    ChainPlan p;
+    const void* g[kMaxLinks];
+};
+
+// Two neighbouring elements of a tile: 16-byte LDS accesses in complex64.
+template <class V>
+struct alignas(16) Pair {
+    V a, b;
+};
+
+// A thread makes the outputs of two neighbouring free parts t.  ADJ: the summed bit (0 or 1
+// of the summed index) at tile position 0, whose two values are neighbours, or -1: then the
+// two t are.
+template <class V, int MODE, int NS, int NB, int ADJ>
+__device__ __forceinline__ void chain_step(const V* in, V* out, const V* gl, const ChainStep& s, int tid) {
+    constexpr int NJ = 1 << NS, NO = 1 << NB;
+    V g[NO][NJ];
+#pragma unroll
+    for (int o = 0; o < NO; ++o)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) g[o][j] = gl[o * 4 + j];
+    const int nf = 1 << (s.lb - NS);
+    const int lo0 = (1 << s.ins[0]) - 1, lo1 = (1 << s.ins[1]) - 1;
+    auto expand = [&](int t) {
+        int x = ((t & ~lo0) << 1) | (t & lo0);
+        if constexpr (NS == 2) x = ((x & ~lo1) << 1) | (x & lo1);
+        return x;
+    };
+    auto pair = [&](int x) { return *reinterpret_cast<const Pair<V>*>(in + x); };
+    for (int t = 2 * tid; t < nf; t += 2 * kChainThreads) {
+        V xs[2][NJ];
+        if constexpr (ADJ >= 0) {
+            constexpr int kAdj = 1 << ADJ, kOther = kAdj == 1 ? 2 : 1;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int x = expand(t + h);
+                const Pair<V> v = pair(x);
+                xs[h][0] = v.a;
+                xs[h][kAdj] = v.b;
+                if constexpr (NS == 2) {
+                    const Pair<V> w = pair(x + s.off[kOther]);
+                    xs[h][kOther] = w.a;
+                    xs[h][3] = w.b;
+                }
+            }
+        } else {
+            const int x = expand(t);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const Pair<V> v = pair(x + s.off[j]);
+                xs[0][j] = v.a;
+                xs[1][j] = v.b;
+            }
+        }
+        Acc<V, MODE> acc[2][NO];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int o = 0; o < NO; ++o) mac<V, MODE>(acc[h][o], xs[h][j], g[o][j]);
+#pragma unroll
+        for (int o = 0; o < NO; ++o)
+            *reinterpret_cast<Pair<V>*>(out + t + o * nf) =
+                Pair<V>{finish<V, MODE>(acc[0][o]), finish<V, MODE>(acc[1][o])};
+    }
+}
+
+template <class V, int MODE, int NS, int ADJ>
+__device__ __forceinline__ void chain_step_nb(const V* in, V* out, const V* gl, const ChainStep& s, int tid) {
+    if (s.nb == 0) chain_step<V, MODE, NS, 0, ADJ>(in, out, gl, s, tid);
+    else if (s.nb == 1) chain_step<V, MODE, NS, 1, ADJ>(in, out, gl, s, tid);
+    else chain_step<V, MODE, NS, 2, ADJ>(in, out, gl, s, tid);
+}
+
+// A pass reads and writes the tensor once in HBM, and each step once in LDS: at 8 steps
+// the two and the multiply-adds take about as long as each other, and two workgroups a CU
+// overlap them in part.  The 48-qubit depth-14 sweep (456 steps on tensors of up to 2^29
+// complex64, 1,517 GB step by step, 181 GB in passes): 271.7 ms with k_thin, 99.6 ms;
+// complex128 544 and 225 ms.  Tiles of 2^11 (four workgroups a CU, shorter passes): 103.8
+// and 292 ms.
+template <class V, int MODE>
+__global__ __launch_bounds__(kChainThreads) void k_chain(const V* __restrict__ X, V* __restrict__ C, ChainArgs a) {
+    constexpr int kTile = (8 << kMaxTileBits) / int(sizeof(V));
+    const ChainPlan& p = a.p;
+    __shared__ V gl[kMaxLinks][16];
+    __shared__ __align__(16) V tiles[2][kTile];
+    V *buf = tiles[0], *alt = tiles[1];
+    const int tid = threadIdx.x;
+    if (tid < p.n_steps * 16) {
+        const ChainStep& s = p.step[tid >> 4];
+        const int o = (tid >> 2) & 3, j = tid & 3;
+        if (o < (1 << s.nb) && j < (1 << s.ns))
+            gl[tid >> 4][tid & 15] = static_cast<const V*>(a.g[tid >> 4])[s.g_free[o] + s.g_small[j]];
+    }
+    const int64_t id = int64_t(blockIdx.x) + int64_t(blockIdx.y) * gridDim.x;
+    int64_t base_in = 0, base_out = 0;
+    for (int i = 0; i < p.n_rest; ++i)
+        if ((id >> i) & 1) {
+            base_in += int64_t(1) << p.rest_in[i];
+            base_out += int64_t(1) << p.rest_out[i];
+        }
+    // 16 bytes per access: P low bits of a tile index are one load's or store's elements
+    // (positions 0 to P - 1 are in the tile on both sides).  Thread bits, then up to
+    // 4 step bits, whose offsets are read before the first load
+    constexpr int P = sizeof(V) == 8 ? 1 : 0, hi = kThreadBits + P, kStepBits = 4;
+    struct alignas(16) Pack {
+        V v[1 << P];
+    };
+    {
+        int64_t off_t = base_in, off_s[kStepBits];
+        for (int b = P; b < hi && b < p.tb_in; ++b)
+            if ((tid >> (b - P)) & 1) off_t += int64_t(1) << p.in_pos[b];
+#pragma unroll
+        for (int k = 0; k < kStepBits; ++k) off_s[k] = hi + k < p.tb_in ? int64_t(1) << p.in_pos[hi + k] : 0;
+        const int n = 1 << p.tb_in;
+        if ((tid << P) < n)
+#pragma unroll 4
+            for (int q = 0; (q << hi) < n; ++q) {
+                int64_t off = off_t;
+#pragma unroll
+                for (int k = 0; k < kStepBits; ++k)
+                    if ((q >> k) & 1) off += off_s[k];
+                *reinterpret_cast<Pack*>(buf + (tid << P) + (q << hi)) = *reinterpret_cast<const Pack*>(X + off);
+            }
+    }
+    __syncthreads();
+    for (int i = 0; i < p.n_steps; ++i) {
+        const ChainStep& s = p.step[i];
+        switch (s.ns * 4 + s.adj) {
+            case 3: chain_step_nb<V, MODE, 1, -1>(buf, alt, gl[i], s, tid); break;
+            case 4: chain_step_nb<V, MODE, 1, 0>(buf, alt, gl[i], s, tid); break;
+            case 7: chain_step_nb<V, MODE, 2, -1>(buf, alt, gl[i], s, tid); break;
+            case 8: chain_step_nb<V, MODE, 2, 0>(buf, alt, gl[i], s, tid); break;
+            default: chain_step_nb<V, MODE, 2, 1>(buf, alt, gl[i], s, tid); break;
+        }
+        V* const t = buf;
+        buf = alt;
+        alt = t;
+        __syncthreads();
+    }
+    int64_t off_t = base_out, off_s[kStepBits];
+    for (int b = P; b < hi && b < p.tb_out; ++b)
+        if ((tid >> (b - P)) & 1) off_t += int64_t(1) << p.out_pos[b];
+#pragma unroll
+    for (int k = 0; k < kStepBits; ++k) off_s[k] = hi + k < p.tb_out ? int64_t(1) << p.out_pos[hi + k] : 0;
+    const int n = 1 << p.tb_out;
+    if ((tid << P) < n)
+#pragma unroll 4
+        for (int q = 0; (q << hi) < n; ++q) {
+            int64_t off = off_t;
+#pragma unroll
+            for (int k = 0; k < kStepBits; ++k)
+                if ((q >> k) & 1) off += off_s[k];
+            *reinterpret_cast<Pack*>(C + off) = *reinterpret_cast<const Pack*>(buf + (tid << P) + (q << hi));
+        }
+}
+
+// Where a bit of the growing tensor comes from: an input position, or a bit that a step added.
+struct Origin {
+    int x;  // input position, -1: added in the chain
+};
+
+// The plan of the first n links (step_desc / step_axes as qt_contract_chain takes them), or
+// false when they cannot share a pass.
+bool plan_chain(int nx, int dl, bool c128, int n, const int32_t* desc, const int32_t* axes, ChainPlan* out) {
+    if (n < 1 || n > kMaxLinks) return false;
+    ChainPlan p;
+    std::memset(&p, 0, sizeof p);
+    p.n_steps = n;
+    // bits of the tensor in position order, through the links
+    std::vector<Origin> bits(static_cast<size_t>(nx));
+    for (int i = 0; i < nx; ++i) bits[size_t(i)].x = i;
+    std::vector<char> active(size_t(nx), 0);  // input bits summed in the chain
+    std::vector<std::vector<int>> summed(static_cast<size_t>(n));  // current positions, ascending
+    const int32_t* ax = axes;
+    for (int s = 0; s < n; ++s) {
+        const int rg = desc[3 * s], k = desc[3 * s + 1], rc = desc[3 * s + 2];
+        const int rx = int(bits.size()) / dl, kb = k * dl, nb = (rg - k) * dl;
+        if (k < 1 || kb > 2 || nb < 0 || nb > 2 || k > rx || rc != rx + rg - 2 * k) return false;
+        const int32_t *px = ax, *pg = ax + k, *fs = ax + 2 * k;
+        ax += 2 * k + rc;
+        std::vector<char> used_x(size_t(rx), 0), used_g(size_t(rg), 0);
+        ChainStep& st = p.step[s];
+        st.ns = kb;
+        st.nb = nb;
+        // digit j of the summed index belongs to pair k - 1 - j (src/Network.h:912-916)
+        int s_x[2] = {0, 0}, s_g[2] = {0, 0};
+        for (int i = 0; i < k; ++i) {
+            if (px[i] < 0 || px[i] >= rx || pg[i] < 0 || pg[i] >= rg || used_x[size_t(px[i])]++ || used_g[size_t(pg[i])]++)
+                return false;
+            for (int t = 0; t < dl; ++t) {
+                s_x[(k - 1 - i) * dl + t] = px[i] * dl + t;
+                s_g[(k - 1 - i) * dl + t] = pg[i] * dl + t;
+            }
+        }
+        for (int b = 0; b < kb; ++b) summed[size_t(s)].push_back(s_x[b]);
+        std::sort(summed[size_t(s)].begin(), summed[size_t(s)].end());
+        for (int j = 0; j < (1 << kb); ++j)
+            for (int b = 0; b < kb; ++b)
+                if ((j >> b) & 1) st.g_small[j] += 1 << s_g[b];
+        // free axes: the tensor's in their order, then the small operand's
+        int prev = -1, f = 0;
+        for (; f < rc && (fs[f] & QT_FROM_A); ++f) {
+            const int axis = fs[f] & ~QT_FROM_A;
+            if (axis <= prev || axis >= rx || used_x[size_t(axis)]++) return false;
+            prev = axis;
+        }
+        if (f != rx - k) return false;
+        int g_bit[2] = {0, 0}, ng = 0;
+        for (; f < rc; ++f) {
+            if ((fs[f] & QT_FROM_A) || fs[f] < 0 || fs[f] >= rg || used_g[size_t(fs[f])]++) return false;
+            for (int t = 0; t < dl; ++t) g_bit[ng++] = fs[f] * dl + t;
+        }
+        for (int o = 0; o < (1 << nb); ++o)
+            for (int b = 0; b < nb; ++b)
+                if ((o >> b) & 1) st.g_free[o] += 1 << g_bit[b];
+        // store the pairs' own order for the offsets below
+        for (int b = 0; b < kb; ++b) st.off[b] = s_x[b];
+        std::vector<Origin> next;
+        for (size_t b = 0; b < bits.size(); ++b) {
+            if (std::find(summed[size_t(s)].begin(), summed[size_t(s)].end(), int(b)) == summed[size_t(s)].end())
+                next.push_back(bits[b]);
+            else if (bits[b].x >= 0)
+                active[size_t(bits[b].x)] = 1;
+        }
+        for (int b = 0; b < nb; ++b) next.push_back(Origin{-1});
+        bits.swap(next);
+    }
+    // the tile: the summed input bits, the four lowest bits of the input (three in
+    // complex128: 128 bytes) and of the result, then the lowest others up to the size that
+    // the largest intermediate allows
+    const int line = c128 ? 3 : 4;
+    std::vector<char> in_tile(active);
+    for (int i = 0; i < line && i < nx; ++i) in_tile[size_t(i)] = 1;
+    for (int i = 0; i < line && i < int(bits.size()); ++i)
+        if (bits[size_t(i)].x >= 0) in_tile[size_t(bits[size_t(i)].x)] = 1;
+    int grow = 0, most = 0;  // the largest excess of an intermediate over the input tile
+    for (int s = 0; s < n; ++s) {
+        grow += p.step[s].nb - p.step[s].ns;
+        most = std::max(most, grow);
+    }
+    int tb = 0;
+    for (char t : in_tile) tb += t;
+    // at least 2^8 tiles where the tensor is small, and a tile that fills the workgroup
+    const int cap = std::min(c128 ? kMaxTileBits - 1 : kMaxTileBits, std::max(9, nx - 8));
+    if (tb + most > cap || tb + grow < 2) return false;
+    for (int i = 0; i < nx && tb + most < cap; ++i)
+        if (!in_tile[size_t(i)]) {
+            in_tile[size_t(i)] = 1;
+            ++tb;
+        }
+    p.tb_in = tb;
+    p.tb_out = tb + grow;
+    int k = 0;
+    for (int i = 0; i < nx; ++i)
+        if (in_tile[size_t(i)]) p.in_pos[k++] = i;
+    k = 0;
+    int r = 0;
+    for (size_t i = 0; i < bits.size(); ++i) {
+        if (bits[i].x < 0 || in_tile[size_t(bits[i].x)]) {
+            p.out_pos[k++] = int(i);
+        } else {
+            p.rest_in[r] = bits[i].x;
+            p.rest_out[r++] = int(i);
+        }
+    }
+    p.n_rest = r;
+    if (k != p.tb_out || r > 48) return false;
+    // tile positions of the summed bits: their rank among the tile's bits at that step
+    std::vector<Origin> cur(static_cast<size_t>(nx));
+    for (int i = 0; i < nx; ++i) cur[size_t(i)].x = i;
+    for (int s = 0; s < n; ++s) {
+        ChainStep& st = p.step[s];
+        std::vector<int> rank_of(cur.size(), -1);
+        int lb = 0;
+        for (size_t b = 0; b < cur.size(); ++b)
+            if (cur[b].x < 0 || in_tile[size_t(cur[b].x)]) rank_of[b] = lb++;
+        st.lb = lb;
+        if (lb - st.ns < 1) return false;  // a thread takes two free parts
+        const int s_x[2] = {st.off[0], st.off[1]};
+        st.adj = -1;
+        for (int b = 0; b < st.ns; ++b)
+            if (rank_of[size_t(s_x[b])] == 0) st.adj = b;
+        for (int i = 0; i < st.ns; ++i) st.ins[i] = rank_of[size_t(summed[size_t(s)][size_t(i)])];
+        std::memset(st.off, 0, sizeof st.off);
+        for (int j = 0; j < (1 << st.ns); ++j)
+            for (int b = 0; b < st.ns; ++b)
+                if ((j >> b) & 1) st.off[j] += 1 << rank_of[size_t(s_x[b])];
+        std::vector<Origin> next;
+        for (size_t b = 0; b < cur.size(); ++b)
+            if (std::find(summed[size_t(s)].begin(), summed[size_t(s)].end(), int(b)) == summed[size_t(s)].end())
+                next.push_back(cur[b]);
+        for (int b = 0; b < st.nb; ++b) next.push_back(Origin{-1});
+        cur.swap(next);
+    }
+    *out = p;
+    return true;
+}
+
+template <class V, int MODE>
+qt_status launch_chain(Ctx* c, const Tensor* X, Tensor* C, const ChainArgs& a) {
+    const int64_t tiles = int64_t(1) << a.p.n_rest;
+    const unsigned gx = unsigned(std::min<int64_t>(tiles, 65536));
+    const unsigned gy = unsigned(tiles / gx);
+    hipLaunchKernelGGL((k_chain<V, MODE>), dim3(gx, gy), dim3(kChainThreads), 0, c->stream,
+                       static_cast<const V*>(X->data), static_cast<V*>(C->data), a);
+    return check_hip(c, hipGetLastError(), "k_chain");
+}
+
+}  // namespace
+
+// Smaller tensors go step by step: their steps take a launch's time each, and a tile per
+// workgroup would leave most of the chip idle.
+constexpr int kChainMinBits = 16;
+
+}  // namespace qt
+
+using qt::set_error;
+
+extern "C" {
+
+int qt_chain_links(int rank_x, int dim_log2, int dtype, int n, const int32_t* desc, const int32_t* axes) {
+    if (n < 1 || !desc || !axes || rank_x < 0 || (dim_log2 != 1 && dim_log2 != 2) || rank_x * dim_log2 > 40 ||
+        rank_x * dim_log2 < qt::kChainMinBits)
+        return 0;
+    for (int m = std::min(n, qt::kMaxLinks); m >= 2; --m) {
+        qt::ChainPlan p;
+        if (qt::plan_chain(rank_x * dim_log2, dim_log2, dtype == QT_DTYPE_C128, m, desc, axes, &p)) return m;
+    }
+    return 0;
+}
+
+qt_status qt_contract_chain(qt_ctx* cx, const qt_tensor* X, int rank_x, int n, const qt_tensor* const* G,
+                            const int32_t* desc, const int32_t* axes, qt_tensor* C, int precision) {
+    if (!cx) return QT_INVALID_INPUT;
+    auto* ctx = &cx->impl;
+    if (!X || !C || !G || !desc || !axes || n < 1 || n > qt::kMaxLinks)
+        return set_error(ctx, QT_INVALID_INPUT, "qt_contract_chain: null argument or too many links");
+    const qt::Tensor& x = X->impl;
+    qt::Tensor& c = C->impl;
+    const bool c128 = x.dtype == QT_DTYPE_C128, rescale = (precision & QT_RESCALE) != 0;
+    const int form = precision & ~QT_RESCALE;
+    if ((c128 && (form != QT_PLAIN_C128 || rescale)) ||
+        (!c128 && form != QT_C64_4M && form != QT_C64_3M && form != QT_C64_BF16X3))
+        return set_error(ctx, QT_INVALID_INPUT, "qt_contract_chain: precision does not fit dtype");
+    if (x.rank != rank_x || c.rank != desc[3 * (n - 1) + 2] || c.dtype != x.dtype || c.dim_log2 != x.dim_log2 || &x == &c)
+        return set_error(ctx, QT_INVALID_INPUT, "qt_contract_chain: C or X does not match the links");
+    qt::ChainArgs a;
+    std::memset(&a, 0, sizeof a);
+    for (int s = 0; s < n; ++s) {
+        if (!G[s] || G[s]->impl.rank != desc[3 * s] || G[s]->impl.dtype != x.dtype ||
+            G[s]->impl.dim_log2 != x.dim_log2 || &G[s]->impl == &c)
+            return set_error(ctx, QT_INVALID_INPUT, "qt_contract_chain: a small tensor does not match its link");
+        if (G[s]->impl.exp_slot >= 0)
+            return set_error(ctx, QT_UNSUPPORTED, "qt_contract_chain: a small tensor carries an exponent");
+        a.g[s] = G[s]->impl.data;
+    }
+    if (!qt::plan_chain(rank_x * x.dim_log2, x.dim_log2, c128, n, desc, axes, &a.p))
+        return set_error(ctx, QT_UNSUPPORTED, "qt_contract_chain: the links do not fit one pass");
+    std::lock_guard<std::recursive_mutex> g(ctx->mu);
+    qt_status s = qt::check_deadline(ctx, "qt_contract_chain");
+    if (s != QT_OK) return s;
+    (void)hipSetDevice(ctx->device);
+    switch (form) {
+        case QT_PLAIN_C128: s = qt::launch_chain<double2, qt::MODE_PLAIN>(ctx, &x, &c, a); break;
+        case QT_C64_4M: s = qt::launch_chain<float2, qt::MODE_4M>(ctx, &x, &c, a); break;
+        case QT_C64_3M: s = qt::launch_chain<float2, qt::MODE_3M>(ctx, &x, &c, a); break;
+        default: s = qt::launch_chain<float2, qt::MODE_BF16X3>(ctx, &x, &c, a); break;
+    }
+    if (s == QT_OK) s = rescale ? qt::rescale_c64(ctx, &x, &G[0]->impl, &c) : qt::carry_exponent(ctx, &x, &G[0]->impl, &c);
+    return s;
+}
+
+}  // extern "C"

@@ -677,18 +677,60 @@ std::complex<double> SlicedNetwork::RunWith(qt_ctx* ctx, int precision, SliceSta
                 for (size_t s = 0; s < steps_.size(); ++s) {
                     if (fuse && step_fused_[s]) continue;
                     const Step& st = steps_[s];
+                    // consecutive steps that each contract the last result (as operand A)
+                    // with another tensor: as many as one pass takes
+                    std::vector<size_t> link{s};
+                    for (size_t q = s + 1; q < steps_.size() && link.size() < 8; ++q) {
+                        if (fuse && step_fused_[q]) continue;
+                        if (steps_[q].a != n_leaves_ + int(link.back()) || !ops[size_t(steps_[q].b)]) break;
+                        link.push_back(q);
+                    }
+                    int taken = 0;
+                    std::vector<int32_t> desc, axes;
+                    if (link.size() > 1) {
+                        for (size_t q : link) {
+                            const Step& l = steps_[q];
+                            desc.insert(desc.end(), {l.rank_b, l.k, l.rank_c});
+                            axes.insert(axes.end(), l.pair_a.begin(), l.pair_a.end());
+                            axes.insert(axes.end(), l.pair_b.begin(), l.pair_b.end());
+                            axes.insert(axes.end(), l.free_src.begin(), l.free_src.end());
+                        }
+                        taken = qt_chain_links(st.rank_a, dl_, dtype, int(link.size()), desc.data(), axes.data());
+                    }
                     qt_tensor* c = nullptr;
-                    CheckQt(ctx, qt_tensor_alloc_empty(ctx, st.rank_c, dl_, dtype, &c), "qt_tensor_alloc_empty");
-                    ops[size_t(n_leaves_) + s] = c;
-                    CheckQt(ctx,
-                            qt_contract_pair(ctx, ops[size_t(st.a)], st.rank_a, ops[size_t(st.b)], st.rank_b, st.k,
-                                             st.pair_a.data(), st.pair_b.data(), st.rank_c, st.free_src.data(), c,
-                                             precision, nullptr),
-                            "qt_contract_pair");
-                    for (int op : {st.a, st.b}) {
+                    if (taken > 0) {
+                        link.resize(size_t(taken));
+                        std::vector<const qt_tensor*> small;
+                        for (size_t q : link) small.push_back(ops[size_t(steps_[q].b)]);
+                        CheckQt(ctx, qt_tensor_alloc_empty(ctx, steps_[link.back()].rank_c, dl_, dtype, &c),
+                                "qt_tensor_alloc_empty");
+                        const qt_status got = qt_contract_chain(ctx, ops[size_t(st.a)], st.rank_a, taken, small.data(),
+                                                                desc.data(), axes.data(), c, precision);
+                        if (got == QT_UNSUPPORTED) {  // a small tensor with an exponent: step by step
+                            qt_tensor_free(ctx, c);
+                            taken = 0;
+                        } else {
+                            ops[size_t(n_leaves_) + link.back()] = c;
+                            CheckQt(ctx, got, "qt_contract_chain");
+                        }
+                    }
+                    if (taken == 0) {
+                        link.resize(1);
+                        CheckQt(ctx, qt_tensor_alloc_empty(ctx, st.rank_c, dl_, dtype, &c), "qt_tensor_alloc_empty");
+                        ops[size_t(n_leaves_) + s] = c;
+                        CheckQt(ctx,
+                                qt_contract_pair(ctx, ops[size_t(st.a)], st.rank_a, ops[size_t(st.b)], st.rank_b, st.k,
+                                                 st.pair_a.data(), st.pair_b.data(), st.rank_c, st.free_src.data(), c,
+                                                 precision, nullptr),
+                                "qt_contract_pair");
+                    }
+                    auto done = [&](int op) {
                         qt_tensor_free(ctx, ops[size_t(op)]);
                         ops[size_t(op)] = nullptr;
-                    }
+                    };
+                    done(st.a);
+                    for (size_t q : link) done(steps_[q].b);
+                    s = link.back();
                 }
                 CheckQt(ctx, qt_tensor_accumulate(ctx, ops.back(), acc), "qt_tensor_accumulate");
                 release();

@@ -1,0 +1,106 @@
+"""Chains of thin steps in one pass (qt_contract_chain) against the same steps through
+qt_contract_pair: the same arithmetic in the same order, so the same bits."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import qtorch_amd as qa
+from qtorch_amd import workloads as wl
+from qtorch_amd._native import _i32, hip
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = qa.Context(0)
+    yield c
+    c.close()
+
+
+# links as (tensor axes summed in the small tensor's order, new axes): counted from the
+# tensor so far; -1 is its last axis
+CHAINS = [
+    (16, 1, [((0, -1), 1), ((-1,), 2)]),                       # the smallest tensor
+    (19, 1, [((0, -1), 1), ((-1,), 2), ((5, -1), 1), ((-1,), 2), ((0, -1), 1), ((0,), 2), ((-1,), 1), ((3,), 0)]),
+    (21, 1, [((20, 4), 2), ((0,), 2), ((0,), 2), ((1, 0), 0)]),
+    (18, 1, [((17,), 2), ((18,), 2), ((19,), 2), ((20, 0), 1)]),  # grows three bits first
+    (9, 2, [((0,), 1), ((8,), 1), ((4,), 1)]),                 # dimension 4, two bits a wire
+    (22, 1, [((2,), 1), ((9,), 1), ((15,), 1), ((21,), 1), ((20,), 1)]),
+]
+
+
+@pytest.mark.parametrize("prec", [qa.QT_PLAIN_C128, qa.QT_C64_4M, qa.QT_C64_3M, qa.QT_C64_BF16X3])
+@pytest.mark.parametrize("rank,d,links", CHAINS)
+def test_chain_equals_steps(ctx, rank, d, links, prec):
+    rng = np.random.default_rng(rank + 10 * len(links) + d)
+    c128 = prec == qa.QT_PLAIN_C128
+    dt, dtype = (np.complex128, qa.QT_DTYPE_C128) if c128 else (np.complex64, qa.QT_DTYPE_C64)
+
+    def tensor(r):
+        v = (rng.standard_normal(1 << (d * r)) + 1j * rng.standard_normal(1 << (d * r))).astype(dt)
+        return qa.Tensor(ctx, r, d, dtype).upload(v)
+
+    x = tensor(rank)
+    steps, small, desc, axes, r = [], [], [], [], rank
+    for pos, new in links:
+        pos = [p % r for p in pos]
+        order = [int(i) for i in rng.permutation(len(pos) + new)]  # the small tensor's axes, shuffled
+        pairs = list(zip(pos, order))
+        free = [(True, i) for i in range(r) if i not in pos] + [(False, a) for a in order[len(pos):]]
+        g = tensor(len(order))
+        steps.append((g, pairs, free))
+        small.append(g)
+        r = len(free)
+        desc += [len(order), len(pos), r]
+        axes += [p for p, _ in pairs] + [q for _, q in pairs]
+        axes += [a | qa.QT_FROM_A if from_a else a for from_a, a in free]
+    n = hip.qt_chain_links(rank, d, dtype, len(links), _i32(desc), _i32(axes))
+    assert n >= 2
+    ref = x
+    for g, pairs, free in steps[:n]:
+        ref, _ = qa.contract_pair(ctx, ref, g, pairs, free, prec)
+    c = qa.Tensor(ctx, desc[3 * n - 1], d, dtype)
+    gs = (ctypes.c_void_p * n)(*[g.handle for g in small[:n]])
+    ctx.check(hip.qt_contract_chain(ctx.handle, x.handle, rank, n, gs, _i32(desc), _i32(axes), c.handle, prec), "chain")
+    assert np.array_equal(c.download(), ref.download()), n
+
+
+def test_what_does_not_chain(ctx):
+    """A small tensor, three summed bits, free axes out of order, the small tensor's axes
+    first: none of them is taken."""
+    def links(rank, per_link):
+        desc, axes = [], []
+        for pairs, free, rg in per_link:
+            desc += [rg, len(pairs), len(free)]
+            axes += [p for p, _ in pairs] + [q for _, q in pairs]
+            axes += [a | qa.QT_FROM_A if from_a else a for from_a, a in free]
+        return hip.qt_chain_links(rank, 1, qa.QT_DTYPE_C64, len(per_link), _i32(desc), _i32(axes))
+
+    def gate(rank, pos, new):
+        return ([(p, i) for i, p in enumerate(pos)],
+                [(True, i) for i in range(rank) if i not in pos] + [(False, len(pos) + i) for i in range(new)],
+                len(pos) + new)
+
+    good = gate(18, (0,), 1)
+    assert links(18, [good, good]) == 2
+    assert links(18, [good]) == 0
+    assert links(15, [gate(15, (0,), 1)] * 2) == 0
+    assert links(18, [gate(18, (0, 1, 2), 2)] * 2) == 0
+    swapped = (good[0], [good[1][1], good[1][0]] + good[1][2:], good[2])
+    assert links(18, [good, swapped]) == 0
+    first = (good[0], good[1][-1:] + good[1][:-1], good[2])
+    assert links(18, [first, good]) == 0
+
+
+def test_sweep_with_chains_matches_line_graph(ctx):
+    """The sweep order of a 20-qubit circuit (its large steps in chains) against the line-graph
+    order of the same circuit, rescaled form included."""
+    q, bits = wl.grid_random_circuit(4, 5, 12, seed=3), wl.bitstring(20, 4)
+    ref, _ = qa.SlicedNetwork(q, bits, dim_log2=1, order=qa.ORDER_LINEGRAPH, max_bits=26).run(ctx)
+    sweep = qa.SlicedNetwork(q, bits, dim_log2=1, order=qa.ORDER_SWEEP, max_bits=28)
+    assert sweep.plan()["peak_bits"] >= 16
+    for prec, tol in ((qa.QT_PLAIN_C128, 1e-11), (qa.QT_C64_4M, 2e-5), (qa.QT_C64_4M | qa.QT_RESCALE, 2e-5)):
+        v, _ = sweep.run(ctx, prec)
+        assert abs(v - ref) <= tol * max(abs(ref), 2.0 ** -10)
