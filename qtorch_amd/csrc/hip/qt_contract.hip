@@ -421,6 +421,10 @@ __global__ __launch_bounds__(kThreads) void k_reduce_final(const V* __restrict__
     if (threadIdx.x == 0) C[c] = part[0];
 }
 
+__device__ __forceinline__ uint16_t bf16_bits(float x) {  // round to nearest even
+    return uint16_t(__float_as_uint(bf16_round(x)) >> 16);
+}
+
 // LDS-staged bit permutation (see PermPlan).  Reads walk the input-low bits
 // contiguously, writes walk the output-low bits contiguously.
 // Tile element t sits at slot t with its low 6 bits xor-ed with its row t / 64: a read
@@ -432,7 +436,9 @@ __global__ __launch_bounds__(kThreads) void k_reduce_final(const V* __restrict__
 // 16-byte ones.
 __device__ __forceinline__ int tile_slot(int t) { return t ^ ((t >> 6) & 63); }
 
-template <class V, int P>
+// SPLIT (complex64, P = 1): out is four bf16 planes of 2^nbits elements (re hi, re lo, im hi,
+// im lo; x = hi + lo, both rounded to nearest), a pair of neighbours one 4-byte store each.
+template <class V, int P, bool SPLIT>
 __global__ __launch_bounds__(kThreads) void k_permute(const V* __restrict__ in, V* __restrict__ out,
                                                       PermPlan p) {
     extern __shared__ unsigned char smem_raw[];
@@ -508,7 +514,17 @@ __global__ __launch_bounds__(kThreads) void k_permute(const V* __restrict__ in, 
                 }
             if constexpr (P == 1) {
                 const V a = tile[tile_slot(t)], b2 = tile[tile_slot(t | pair_bit)];
-                *reinterpret_cast<float4*>(out + off) = make_float4(a.x, a.y, b2.x, b2.y);
+                if constexpr (SPLIT) {
+                    uint32_t* const o = reinterpret_cast<uint32_t*>(out) + (off >> 1);
+                    const int64_t plane = int64_t(1) << (p.nbits - 1);
+                    auto two = [](float x, float y) { return uint32_t(bf16_bits(x)) | uint32_t(bf16_bits(y)) << 16; };
+                    o[0] = two(a.x, b2.x);
+                    o[plane] = two(a.x - bf16_round(a.x), b2.x - bf16_round(b2.x));
+                    o[2 * plane] = two(a.y, b2.y);
+                    o[3 * plane] = two(a.y - bf16_round(a.y), b2.y - bf16_round(b2.y));
+                } else {
+                    *reinterpret_cast<float4*>(out + off) = make_float4(a.x, a.y, b2.x, b2.y);
+                }
             } else {
                 out[off] = tile[tile_slot(t)];
             }
@@ -661,10 +677,6 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm_c128(const double2* __rest
 constexpr int HK = 32;
 typedef float f4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ uint16_t bf16_bits(float x) {  // round to nearest even
-    return uint16_t(__float_as_uint(bf16_round(x)) >> 16);
-}
 
 template <int MODE>
 __global__ __launch_bounds__(kThreads) void k_gemm_c64(const float2* __restrict__ Ap, const float2* __restrict__ Bp,
@@ -1131,12 +1143,23 @@ qt_status run_permute(Ctx* c, const V* in, V* out, const PermPlan& p) {
                        (reinterpret_cast<uintptr_t>(out) & 15) == 0;
     if constexpr (sizeof(V) == 8) {
         if (pairs) {
-            hipLaunchKernelGGL((k_permute<V, 1>), dim3(gx, gy), dim3(kThreads), lds, c->stream, in, out, p);
+            hipLaunchKernelGGL((k_permute<V, 1, false>), dim3(gx, gy), dim3(kThreads), lds, c->stream, in, out, p);
             return check_hip(c, hipGetLastError(), "k_permute");
         }
     }
-    hipLaunchKernelGGL((k_permute<V, 0>), dim3(gx, gy), dim3(kThreads), lds, c->stream, in, out, p);
+    hipLaunchKernelGGL((k_permute<V, 0, false>), dim3(gx, gy), dim3(kThreads), lds, c->stream, in, out, p);
     return check_hip(c, hipGetLastError(), "k_permute");
+}
+
+// in -> four bf16 planes in `out` (2^nbits elements of 8 bytes in all)
+qt_status run_permute_split(Ctx* c, const float2* in, void* out, const PermPlan& p) {
+    const int64_t blocks = int64_t(1) << p.n_rest;
+    const unsigned gx = unsigned(blocks < 65536 ? blocks : 65536);
+    const unsigned gy = unsigned((blocks + gx - 1) / gx);
+    const size_t lds = (size_t(1) << (p.tl + p.n_extra_in)) * sizeof(float2);
+    hipLaunchKernelGGL((k_permute<float2, 1, true>), dim3(gx, gy), dim3(kThreads), lds, c->stream, in,
+                       static_cast<float2*>(out), p);
+    return check_hip(c, hipGetLastError(), "k_permute (split)");
 }
 
 bool is_identity(const int* src, int n) {
@@ -1387,6 +1410,117 @@ __global__ __launch_bounds__(kThreads, MODE == MODE_3M ? 1 : 2) void k_gemm_c64_
             }
 }
 
+// Large bf16x3 GEMMs: the permutes write the operands as bf16 planes in the order that an
+// MFMA lane reads, plane[k / 8][row][k % 8], so a k-tile goes to LDS and from LDS to the
+// matrix cores in 16-byte pieces without any conversion (k_gemm_c64 splits every element
+// again for each tile that reads it, in 2-byte LDS writes: 235 million bank-conflict cycles
+// on the product below).  128 x 128 outputs, four waves of 64 x 64, k-tiles of 32 in two LDS
+// buffers; same products in the same order as k_gemm_c64.
+constexpr int kPlaneTile = 4 * BT;  // 16-byte pieces of one plane of a k-tile: [k / 8][row]
+
+__global__ __launch_bounds__(kThreads, 1) void k_gemm_bf16x3(const uint4* __restrict__ Ap, const uint4* __restrict__ Bp,
+                                                             float2* __restrict__ C, int64_t M, int64_t N, int64_t K,
+                                                             int64_t k_all) {
+    __shared__ uint4 lds[2][2][4 * kPlaneTile];  // [buffer][operand][plane][k / 8][row]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = wave & 1, wn = wave >> 1;
+    const int li = lane & 15, lk = lane >> 4;
+    const int64_t tiles_m = M / BT;
+    const int64_t tile = int64_t(blockIdx.x) + int64_t(blockIdx.y) * gridDim.x;
+    if (tile >= tiles_m * (N / BT)) return;
+    int64_t tm, tn;
+    gemm_tile(tile, tiles_m, N / BT, tm, tn);
+    const int64_t m0 = tm * BT, n0 = tn * BT;
+    // split K: workgroups with blockIdx.z = z take summed rows [z K, (z + 1) K) and write
+    // their own M x N partial product at C + z M N
+    const int64_t k8_0 = int64_t(blockIdx.z) * (K / 8);
+    C += int64_t(blockIdx.z) * M * N;
+    f4_t acc_re[4][4], acc_im[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc_re[i][j] = acc_im[i][j] = f4_t{0, 0, 0, 0};
+    // a thread moves piece tid + 256 q of each plane: k / 8 = tid / 128 + 2 q, row tid % 128
+    typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
+    u4_t ra[4][2], rb[4][2];
+    const u4_t* pa = reinterpret_cast<const u4_t*>(Ap) + (k8_0 + (tid >> 7)) * M + m0 + (tid & 127);
+    const u4_t* pb = reinterpret_cast<const u4_t*>(Bp) + (k8_0 + (tid >> 7)) * N + n0 + (tid & 127);
+    const int64_t plane_a = k_all / 8 * M, plane_b = k_all / 8 * N;
+    auto fetch = [&]() {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                ra[q][h] = pa[q * plane_a + 2 * h * M];
+                rb[q][h] = pb[q * plane_b + 2 * h * N];
+            }
+        pa += 4 * M;
+        pb += 4 * N;
+    };
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                *reinterpret_cast<u4_t*>(&lds[buf][0][q * kPlaneTile + tid + kThreads * h]) = ra[q][h];
+                *reinterpret_cast<u4_t*>(&lds[buf][1][q * kPlaneTile + tid + kThreads * h]) = rb[q][h];
+            }
+    };
+    auto frag = [&](int buf, int op, int q, int row) {
+        return *reinterpret_cast<const bf8_t*>(&lds[buf][op][q * kPlaneTile + lk * BT + row]);
+    };
+    auto neg = [](bf8_t v) {
+        u4_t u = *reinterpret_cast<u4_t*>(&v);
+        u ^= 0x80008000u;
+        return *reinterpret_cast<bf8_t*>(&u);
+    };
+    fetch();
+    stage(0);
+    __syncthreads();
+    int buf = 0;
+    for (int64_t k0 = 0; k0 < K; k0 += HK, buf ^= 1) {
+        const bool more = k0 + HK < K;
+        if (more) fetch();
+        bf8_t a[4][4];
+#pragma unroll
+        for (int bm = 0; bm < 4; ++bm)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) a[bm][q] = frag(buf, 0, q, wm * 64 + bm * 16 + li);
+        // re += br ar - bi ai; im += bi ar + br ai, each product hi*hi + hi*lo + lo*hi: (B
+        // operand, A operand) per round, 4 and 5 being -im hi and -im lo
+        constexpr int kRe[6][2] = {{0, 0}, {0, 1}, {1, 0}, {4, 2}, {4, 3}, {5, 2}};
+        constexpr int kIm[6][2] = {{2, 0}, {2, 1}, {3, 0}, {0, 2}, {0, 3}, {1, 2}};
+#pragma unroll
+        for (int bn = 0; bn < 4; ++bn) {
+            bf8_t b[6];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) b[q] = frag(buf, 1, q, wn * 64 + bn * 16 + li);
+            b[4] = neg(b[2]);
+            b[5] = neg(b[3]);
+#pragma unroll
+            for (int t = 0; t < 6; ++t)
+#pragma unroll
+                for (int bm = 0; bm < 4; ++bm) {
+                    acc_re[bn][bm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[kRe[t][0]], a[bm][kRe[t][1]],
+                                                                             acc_re[bn][bm], 0, 0, 0);
+                    acc_im[bn][bm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[kIm[t][0]], a[bm][kIm[t][1]],
+                                                                             acc_im[bn][bm], 0, 0, 0);
+                }
+        }
+        if (more) stage(buf ^ 1);  // read last in the k-tile before, behind its barrier
+        __syncthreads();
+    }
+#pragma unroll
+    for (int bn = 0; bn < 4; ++bn)
+#pragma unroll
+        for (int bm = 0; bm < 4; ++bm)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int64_t n = n0 + wn * 64 + bn * 16 + 4 * lk + r;
+                C[m0 + wm * 64 + bm * 16 + li + M * n] = float2{acc_re[bn][bm][r], acc_im[bn][bm][r]};
+            }
+}
+
 // Largest |re|, |im| of a complex64 tensor in two launches and no atomics: each
 // workgroup of k_absmax_c64 writes the maximum of its grid-stride share to parts[];
 // every workgroup of k_rescale_c64 reduces the (at most kAbsParts) partial maxima
@@ -1572,7 +1706,26 @@ qt_status run_gemm(Ctx* c, const Tensor* A, const Tensor* B, Tensor* C, const Bi
     const V* bp = static_cast<const V*>(B->data);
     void* abuf = nullptr;
     void* bbuf = nullptr;
-    const bool perm_a = !is_identity(src_a, mbits + sb), perm_b = !is_identity(src_b, nbits_n + sb);
+    bool perm_a = !is_identity(src_a, mbits + sb), perm_b = !is_identity(src_b, nbits_n + sb);
+    // bf16x3 with whole 128 x 128 x 32 tiles: the permutes write bf16 planes, the lowest
+    // three summed bits first (k_gemm_bf16x3).  Each operand then needs scratch of its own
+    // size, also one that is in place, so not with a caller's workspace
+    const bool planes = MODE == MODE_BF16X3 && !ws && mbits >= 7 && nbits_n >= 7 && sb >= 5;
+    if (planes) {
+        auto lowest_first = [&](int* src, int free_bits, const uint8_t* sum) {
+            for (int j = free_bits - 1; j >= 0; --j) src[j + 3] = src[j];
+            for (int j = 0; j < 3; ++j) src[j] = sum[j];
+        };
+        lowest_first(src_a, mbits, m.s_a);
+        lowest_first(src_b, nbits_n, m.s_b);
+        perm_a = perm_b = true;
+    }
+    auto rewrite = [&](const Tensor* t, void* out, int nbits, const int* src) {
+        const PermPlan p = make_perm_plan(nbits, src, kPermTileBits);
+        if constexpr (MODE == MODE_BF16X3)
+            if (planes) return run_permute_split(c, static_cast<const float2*>(t->data), out, p);
+        return permute(c, t->data, out, t->dtype, p);
+    };
     // a workspace holds A's permute at its start and B's after it (256-byte aligned)
     const size_t ws_b = perm_a ? (A->bytes + 255) / 256 * 256 : 0;
     if (ws && ws_b + (perm_b ? B->bytes : 0) > ws->bytes)
@@ -1582,7 +1735,7 @@ qt_status run_gemm(Ctx* c, const Tensor* A, const Tensor* B, Tensor* C, const Bi
         hipError_t e = hipSuccess;
         abuf = ws ? static_cast<void*>(ws->base) : c->pool.alloc(A->bytes, &e);
         if (!abuf) return check_hip(c, e, "gemm scratch A");
-        s = permute(c, A->data, abuf, A->dtype, make_perm_plan(mbits + sb, src_a, kPermTileBits));
+        s = rewrite(A, abuf, mbits + sb, src_a);
         ap = static_cast<const V*>(abuf);
     }
     if (s == QT_OK && perm_b) {
@@ -1592,7 +1745,7 @@ qt_status run_gemm(Ctx* c, const Tensor* A, const Tensor* B, Tensor* C, const Bi
             if (!ws) c->pool.release(abuf);
             return check_hip(c, e, "gemm scratch B");
         }
-        s = permute(c, B->data, bbuf, B->dtype, make_perm_plan(nbits_n + sb, src_b, kPermTileBits));
+        s = rewrite(B, bbuf, nbits_n + sb, src_b);
         bp = static_cast<const V*>(bbuf);
     }
     if (s == QT_OK) {
@@ -1629,42 +1782,45 @@ qt_status run_gemm(Ctx* c, const Tensor* A, const Tensor* B, Tensor* C, const Bi
             }
         } else {
             bool done = false;
-            if constexpr (MODE == MODE_4M || MODE == MODE_3M) {
-                if (M >= BT && N >= BT && K % BK == 0) {
-                    const int64_t big = (M / BT) * (N / BT);
-                    const unsigned bx = unsigned(big < 65536 ? big : 65536);
-                    const unsigned by = unsigned((big + bx - 1) / bx);
-                    // fewer output tiles than two per CU: split K (at least kSplitRows
-                    // summed rows per split) into S partial products, then add them in
-                    // order; not with a caller's workspace, which holds no room for them
-                    int S = 1;
-                    if (!ws)
-                        while (big * S < 512 && K / (2 * S) >= kSplitRows && S < 64) S *= 2;
-                    float2* part = nullptr;
-                    if (S > 1) {
-                        hipError_t e = hipSuccess;
-                        part = static_cast<float2*>(c->pool.alloc(size_t(S) * size_t(M * N) * sizeof(float2), &e));
-                        if (!part) {
-                            (void)hipGetLastError();  // no room: one product, unsplit
-                            S = 1;
-                        }
+            if ((MODE == MODE_BF16X3 ? planes : K % BK == 0) && M >= BT && N >= BT) {
+                const int64_t big = (M / BT) * (N / BT);
+                const unsigned bx = unsigned(big < 65536 ? big : 65536);
+                const unsigned by = unsigned((big + bx - 1) / bx);
+                // fewer output tiles than two per CU: split K (at least kSplitRows
+                // summed rows per split) into S partial products, then add them in
+                // order; not with a caller's workspace, which holds no room for them
+                int S = 1;
+                if (!ws)
+                    while (big * S < 512 && K / (2 * S) >= kSplitRows && S < 64) S *= 2;
+                float2* part = nullptr;
+                if (S > 1) {
+                    hipError_t e = hipSuccess;
+                    part = static_cast<float2*>(c->pool.alloc(size_t(S) * size_t(M * N) * sizeof(float2), &e));
+                    if (!part) {
+                        (void)hipGetLastError();  // no room: one product, unsplit
+                        S = 1;
                     }
-                    float2* out = S > 1 ? part : static_cast<float2*>(C->data);
+                }
+                float2* out = S > 1 ? part : static_cast<float2*>(C->data);
+                if constexpr (MODE == MODE_BF16X3)
+                    hipLaunchKernelGGL(k_gemm_bf16x3, dim3(bx, by, unsigned(S)), dim3(kThreads), 0, c->stream,
+                                       reinterpret_cast<const uint4*>(ap), reinterpret_cast<const uint4*>(bp), out, M,
+                                       N, K / S, K);
+                else
                     hipLaunchKernelGGL((k_gemm_c64_big<MODE>), dim3(bx, by, unsigned(S)), dim3(kThreads), 0, c->stream,
                                        ap, bp, out, M, N, K / S);
-                    s = check_hip(c, hipGetLastError(), "k_gemm_c64_big");
-                    if (S > 1) {
-                        const int64_t n4 = M * N / 2;
-                        if (s == QT_OK) {
-                            hipLaunchKernelGGL(k_sum_splits, dim3(unsigned((n4 + kThreads - 1) / kThreads)),
-                                               dim3(kThreads), 0, c->stream, reinterpret_cast<const float4*>(part),
-                                               reinterpret_cast<float4*>(C->data), n4, S);
-                            s = check_hip(c, hipGetLastError(), "k_sum_splits");
-                        }
-                        c->pool.release(part);
+                s = check_hip(c, hipGetLastError(), "k_gemm_c64_big");
+                if (S > 1) {
+                    const int64_t n4 = M * N / 2;
+                    if (s == QT_OK) {
+                        hipLaunchKernelGGL(k_sum_splits, dim3(unsigned((n4 + kThreads - 1) / kThreads)),
+                                           dim3(kThreads), 0, c->stream, reinterpret_cast<const float4*>(part),
+                                           reinterpret_cast<float4*>(C->data), n4, S);
+                        s = check_hip(c, hipGetLastError(), "k_sum_splits");
                     }
-                    done = true;
+                    c->pool.release(part);
                 }
+                done = true;
             }
             if (!done) {
                 // fewer than 512 tiles (64 x 64 here): split K as above
