@@ -322,13 +322,18 @@ class Tensor:
     """A device tensor (qt_tensor): D^rank interleaved complex values."""
 
     def __init__(self, ctx: Context, rank: int, dim_log2: int = 2, dtype: int = QT_DTYPE_C128):
+        self._alloc(ctx, rank, dim_log2, dtype, hip.qt_tensor_alloc, "qt_tensor_alloc")
+
+    def _alloc(self, ctx, rank, dim_log2, dtype, alloc, what) -> "Tensor":
+        self.handle = None
         self.ctx = ctx
         self.rank = rank
         self.dim_log2 = dim_log2
         self.dtype = dtype
         h = _vp()
-        ctx.check(hip.qt_tensor_alloc(ctx.handle, rank, dim_log2, dtype, ctypes.byref(h)), "qt_tensor_alloc")
+        ctx.check(alloc(ctx.handle, rank, dim_log2, dtype, ctypes.byref(h)), what)
         self.handle = h
+        return self
 
     @property
     def np_dtype(self):
@@ -386,7 +391,9 @@ def _i32(vals: Sequence[int]):
 def contract_pair(ctx: Context, a: Tensor, b: Tensor, pairs: Sequence[Tuple[int, int]],
                   free: Sequence[Tuple[bool, int]], precision: int = QT_PLAIN_C128) -> Tuple[Tensor, int]:
     """qt_contract_pair: C = contraction of A and B (Network::ContractIndices semantics)."""
-    c = Tensor(ctx, len(free), a.dim_log2, a.dtype)
+    # every element of C is written: no zero fill (a launch, and a pass over C)
+    c = Tensor.__new__(Tensor)._alloc(ctx, len(free), a.dim_log2, a.dtype, hip.qt_tensor_alloc_empty,
+                                      "qt_tensor_alloc_empty")
     pa = _i32([p[0] for p in pairs])
     pb = _i32([p[1] for p in pairs])
     fs = _i32([(ax | QT_FROM_A) if from_a else ax for from_a, ax in free])

@@ -85,9 +85,9 @@ inline size_t elem_bytes(int dtype) { return dtype == QT_DTYPE_C128 ? 16 : 8; }
 struct BitMap {
     int32_t nbits_c = 0;
     int32_t nbits_s = 0;
-    uint8_t c_src[64];
-    uint8_t s_a[64];
-    uint8_t s_b[64];
+    alignas(8) uint8_t c_src[64];
+    alignas(8) uint8_t s_a[64];
+    alignas(8) uint8_t s_b[64];
 };
 
 // Generic bit permutation for the permute kernel: output bit j <- input bit src[j].
