@@ -137,7 +137,9 @@ qt_status qt_contract_pair(qt_ctx* ctx, const qt_tensor* A, int rank_a, const qt
  * needs to start at zero; calls that overlap on one GPU (from several contexts or
  * threads) race on it.  A GEMM-shaped step with fewer than 512 output tiles and at
  * least 512 summed indices does not split its summed range here (qt_contract_pair
- * does), so its result can differ from qt_contract_pair's in the last bits. */
+ * does), and a sum of 2^9 or more terms into at most 2^16 outputs splits here only from
+ * 2^13 terms into at most 64 outputs, so results can differ from qt_contract_pair's in
+ * the last bits. */
 qt_status qt_contract_pair_noalloc(qt_ctx* ctx, const qt_tensor* A, int rank_a, const qt_tensor* B,
                                    int rank_b, int k, const int32_t* pair_a, const int32_t* pair_b,
                                    int rank_c, const int32_t* free_src, qt_tensor* C, int precision,

@@ -1924,7 +1924,11 @@ inline bool skinny_shape(const BitMap& m, bool split, int mbits) {
 // outputs over 2^12 summed indices (a state projected on 12 qubits, complex64) took
 // 1,244 us on k_skinny, 2^7 over 2^15 (complex128) 389 us on k_direct; here about 50 and
 // 20 us.
-inline bool reduce_shape(const BitMap& m) {
+// With a caller's workspace only the sums that have always split (2^6 outputs, 2^13 terms)
+// do: the others need no scratch on k_direct and k_skinny, and calls that share the
+// workspace may overlap there.
+inline bool reduce_shape(const BitMap& m, const Workspace* ws) {
+    if (ws) return m.nbits_s >= 13 && m.nbits_c <= 6;
     return (m.nbits_s >= 11 && m.nbits_c <= 16) || (m.nbits_s >= 9 && m.nbits_c <= 11);
 }
 
@@ -1934,7 +1938,7 @@ qt_status dispatch_small(Ctx* c, const Tensor* A, const Tensor* B, Tensor* C, co
     const V* a = static_cast<const V*>(A->data);
     const V* b = static_cast<const V*>(B->data);
     V* cc = static_cast<V*>(C->data);
-    if (reduce_shape(m)) return run_reduce<V, MODE>(c, a, b, cc, m, ws);
+    if (reduce_shape(m, ws)) return run_reduce<V, MODE>(c, a, b, cc, m, ws);
     if (skinny_shape(m, split, mbits)) return run_skinny<V, MODE>(c, a, b, cc, m, mbits);
     return run_direct<V, MODE>(c, a, b, cc, m);
 }
