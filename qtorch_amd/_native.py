@@ -716,7 +716,7 @@ class QaoaBatch(_DeviceBatch):
 
     def results(self):
         """(energies, per-edge <ZZ>); the second is None after group-sums-only launches."""
-        e = np.zeros(self.n_sets)
+        e = np.empty(self.n_sets)  # written in full
         if getattr(self, "_sums_only", False):
             _host_check(host.qth_qaoa_batch_results(self.handle, e.ctypes.data_as(_dp), None))
             return e, None

@@ -1097,6 +1097,27 @@ qt_status after_specialised_drop(qt_batch* b) {
     return b->graph_exec ? configure_scratch(b) : QT_OK;  // the captured graph runs the dropped kernel
 }
 
+// Pinned host memory of at least `bytes` for one call under the context's lock, or null
+// (more than 16 MiB, or none to be had): kept by the context, freed with it.
+char* results_stage(Ctx* c, size_t bytes) {
+    constexpr size_t kMost = size_t(16) << 20;
+    if (bytes > kMost) return nullptr;
+    if (c->results_bytes < bytes) {
+        size_t cap = size_t(64) << 10;
+        while (cap < bytes) cap <<= 1;
+        if (c->results) (void)hipHostFree(c->results);
+        c->results = nullptr;
+        c->results_bytes = 0;
+        if (hipHostMalloc(&c->results, cap) != hipSuccess) {
+            (void)hipGetLastError();
+            c->results = nullptr;
+            return nullptr;
+        }
+        c->results_bytes = cap;
+    }
+    return static_cast<char*>(c->results);
+}
+
 qt_status flush_sums(qt_batch* b) {
     if (!b->sums_pending) return QT_OK;
     b->sums_pending = false;
@@ -1605,11 +1626,28 @@ qt_status qt_batch_results(qt_batch* b, double* values, double* group_sums) {
     if (values && !b->values_valid)
         return set_error(ctx, QT_INVALID_INPUT, "qt_batch_results: group-sums-only launches keep no per-instance values");
     qt_status s = qt::flush_sums(b);
+    const size_t value_bytes = values ? size_t(b->n_inst) * 16 : 0;
+    const size_t sum_bytes = group_sums ? size_t(b->n_groups) * 8 : 0;
+    // the status word, the values and the sums in one go: copies to pinned memory queued
+    // behind the launch and one wait for all of them.  Larger results are copied directly
+    char* stage = s == QT_OK ? qt::results_stage(ctx, 256 + value_bytes + sum_bytes) : nullptr;
+    auto fetch = [&](size_t at, void* dst, const void* src, size_t bytes, const char* what) {
+        if (s != QT_OK || bytes == 0) return;
+        s = stage ? check_hip(ctx, hipMemcpyAsync(stage + at, src, bytes, hipMemcpyDeviceToHost, ctx->stream), what)
+                  : check_hip(ctx, hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost), what);
+    };
+    int bad = 0;
+    const bool check = b->params_unchecked;
+    if (stage) {
+        if (check) fetch(0, nullptr, b->d_param_status, sizeof bad, "status");
+        fetch(256, nullptr, b->d_out, value_bytes, "results");
+        fetch(256 + value_bytes, nullptr, b->d_group, sum_bytes, "group sums");
+    }
     if (s == QT_OK) s = check_hip(ctx, hipStreamSynchronize(ctx->stream), "batch sync");
     if (s == QT_OK) b->in_use = false;
-    if (s == QT_OK && b->params_unchecked) {
-        int bad = 0;
-        s = check_hip(ctx, hipMemcpy(&bad, b->d_param_status, sizeof bad, hipMemcpyDeviceToHost), "status");
+    if (s == QT_OK && check) {
+        if (stage) std::memcpy(&bad, stage, sizeof bad);
+        else fetch(0, &bad, b->d_param_status, sizeof bad, "status");
         b->params_unchecked = false;
         if (s == QT_OK && bad) {
             s = qt::launch_fill_zero(ctx, b->d_param_status, 256);
@@ -1618,11 +1656,14 @@ qt_status qt_batch_results(qt_batch* b, double* values, double* group_sums) {
                              "supported range (0, or magnitude in [1e-16, 1e15))");
         }
     }
-    if (s == QT_OK && values && b->n_inst > 0)
-        s = check_hip(ctx, hipMemcpy(values, b->d_out, size_t(b->n_inst) * 16, hipMemcpyDeviceToHost), "results");
-    if (s == QT_OK && group_sums && b->n_groups > 0)
-        s = check_hip(ctx, hipMemcpy(group_sums, b->d_group, size_t(b->n_groups) * 8, hipMemcpyDeviceToHost),
-                      "group sums");
+    if (s != QT_OK) return s;
+    if (stage) {
+        if (value_bytes) std::memcpy(values, stage + 256, value_bytes);
+        if (sum_bytes) std::memcpy(group_sums, stage + 256 + value_bytes, sum_bytes);
+    } else {
+        fetch(0, values, b->d_out, value_bytes, "results");
+        fetch(0, group_sums, b->d_group, sum_bytes, "group sums");
+    }
     return s;
 }
 

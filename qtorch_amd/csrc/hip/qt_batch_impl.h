@@ -230,6 +230,8 @@ bool specialised_consts_change(const qt_batch* b, int64_t offset, const double* 
 // the generated kernel's assumptions on parameter blocks hold for the current
 // instances and the pool's host mirror
 bool specialised_params_hold(const qt_batch* b);
+// pinned host memory for one call's results (qt_batch.hip)
+char* results_stage(Ctx* c, size_t bytes);
 // waits for the batch's queued work before its device arrays are replaced (qt_batch.hip);
 // a batch that has queued nothing since the last wait returns at once
 void quiesce(qt_batch* b);

@@ -48,6 +48,9 @@ struct Ctx {
     hipEvent_t staging_ev[2] = {nullptr, nullptr};
     bool staging_pending[2] = {false, false};
     int staging_next = 0;
+    // pinned host memory that batch results pass through
+    void* results = nullptr;
+    size_t results_bytes = 0;
     // tensors and batches alive on this context: it is not destroyed under them
     int64_t live = 0;
     // power-of-two exponents of rescaled complex64 tensors (value = data * 2^exp)

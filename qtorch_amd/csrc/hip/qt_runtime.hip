@@ -154,6 +154,7 @@ qt_status qt_ctx_destroy(qt_ctx* c) {
         if (c->impl.partials) (void)hipFree(c->impl.partials);
         if (c->impl.d_exp) (void)hipFree(c->impl.d_exp);
         if (c->impl.d_absmax) (void)hipFree(c->impl.d_absmax);
+        if (c->impl.results) (void)hipHostFree(c->impl.results);
         for (int k = 0; k < 2; ++k) {
             if (c->impl.staging[k]) (void)hipHostFree(c->impl.staging[k]);
             if (c->impl.staging_ev[k]) (void)hipEventDestroy(c->impl.staging_ev[k]);
