@@ -158,8 +158,11 @@ qt_status qt_contract_pair_noalloc(qt_ctx* ctx, const qt_tensor* A, int rank_a, 
  * qt_contract_chain runs exactly n such links (QT_UNSUPPORTED if they do not fit a pass, or
  * if a small tensor carries a power-of-two exponent) into C, a distinct, allocated tensor
  * of the last link's rank.  Every step has qt_contract_pair's arithmetic and order, so
- * without QT_RESCALE the result equals the steps one by one bit for bit; with it, C is
- * scaled once, after the last link.  Asynchronous on the context's stream. */
+ * the result equals the steps one by one bit for bit (with QT_RESCALE wherever neither
+ * goes through a subnormal).  With QT_RESCALE C is scaled as by qt_contract_pair, and the
+ * values between the links keep FP32's range as they do step by step: a tile whose largest
+ * value leaves [2^-16, 2^16] is scaled by a power of two on the way.  Asynchronous on the
+ * context's stream. */
 int qt_chain_links(int rank_x, int dim_log2, int dtype, int n, const int32_t* desc, const int32_t* axes);
 qt_status qt_contract_chain(qt_ctx* ctx, const qt_tensor* X, int rank_x, int n, const qt_tensor* const* G,
                             const int32_t* desc, const int32_t* axes, qt_tensor* C, int precision);

@@ -7,7 +7,12 @@
 // and of the lowest bits (whole cache lines), runs the steps on it there, and writes the
 // result's tile.  Each step does k_thin's arithmetic in its order, so the results have
 // the bits that the steps one by one give.
+//
+// Rescaled passes keep their range between the steps: a tile whose largest value leaves
+// [2^-16, 2^16] is scaled by a power of two in LDS (k_chain), and k_chain_scale brings
+// the tiles to the result's one exponent afterwards.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <vector>
 
@@ -53,11 +58,39 @@ struct alignas(16) Pair {
     V a, b;
 };
 
+// Largest |re|, |im| so far; infinite once a value is, NaN passed over.
+template <class V>
+__device__ __forceinline__ void grow_max(float& m, V v) {
+    m = fmaxf(m, fmaxf(fabsf(float(v.x)), fabsf(float(v.y))));
+}
+
+// Largest over the workgroup (lds: one float per wave).
+__device__ __forceinline__ float tile_max(float m, float* lds) {
+    for (int d = 32; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = lds[0];
+    for (int w = 1; w < kChainThreads / 64; ++w) m = fmaxf(m, lds[w]);
+    return m;
+}
+
+// The same over the finite values of a tile.
+__device__ __forceinline__ float tile_max_finite(const float2* t, int n, float* lds) {
+    float m = 0.0f;
+    for (int i = threadIdx.x; i < n; i += kChainThreads) {
+        const float x = fabsf(t[i].x), y = fabsf(t[i].y);
+        if (x < INFINITY) m = fmaxf(m, x);
+        if (y < INFINITY) m = fmaxf(m, y);
+    }
+    return tile_max(m, lds);
+}
+
 // A thread makes the outputs of two neighbouring free parts t.  ADJ: the summed bit (0 or 1
 // of the summed index) at tile position 0, whose two values are neighbours, or -1: then the
 // two t are.
-template <class V, int MODE, int NS, int NB, int ADJ>
-__device__ __forceinline__ void chain_step(const V* in, V* out, const V* gl, const ChainStep& s, int tid) {
+// SCALED: m grows to the outputs' largest |re|, |im|.
+template <class V, int MODE, bool SCALED, int NS, int NB, int ADJ>
+__device__ __forceinline__ void chain_step(const V* in, V* out, const V* gl, const ChainStep& s, int tid, float& m) {
     constexpr int NJ = 1 << NS, NO = 1 << NB;
     V g[NO][NJ];
 #pragma unroll
@@ -105,18 +138,31 @@ __device__ __forceinline__ void chain_step(const V* in, V* out, const V* gl, con
 #pragma unroll
                 for (int o = 0; o < NO; ++o) mac<V, MODE>(acc[h][o], xs[h][j], g[o][j]);
 #pragma unroll
-        for (int o = 0; o < NO; ++o)
-            *reinterpret_cast<Pair<V>*>(out + t + o * nf) =
-                Pair<V>{finish<V, MODE>(acc[0][o]), finish<V, MODE>(acc[1][o])};
+        for (int o = 0; o < NO; ++o) {
+            const Pair<V> v{finish<V, MODE>(acc[0][o]), finish<V, MODE>(acc[1][o])};
+            if constexpr (SCALED) {
+                grow_max(m, v.a);
+                grow_max(m, v.b);
+            }
+            *reinterpret_cast<Pair<V>*>(out + t + o * nf) = v;
+        }
     }
 }
 
-template <class V, int MODE, int NS, int ADJ>
-__device__ __forceinline__ void chain_step_nb(const V* in, V* out, const V* gl, const ChainStep& s, int tid) {
-    if (s.nb == 0) chain_step<V, MODE, NS, 0, ADJ>(in, out, gl, s, tid);
-    else if (s.nb == 1) chain_step<V, MODE, NS, 1, ADJ>(in, out, gl, s, tid);
-    else chain_step<V, MODE, NS, 2, ADJ>(in, out, gl, s, tid);
+template <class V, int MODE, bool SCALED, int NS, int ADJ>
+__device__ __forceinline__ void chain_step_nb(const V* in, V* out, const V* gl, const ChainStep& s, int tid,
+                                              float& m) {
+    if (s.nb == 0) chain_step<V, MODE, SCALED, NS, 0, ADJ>(in, out, gl, s, tid, m);
+    else if (s.nb == 1) chain_step<V, MODE, SCALED, NS, 1, ADJ>(in, out, gl, s, tid, m);
+    else chain_step<V, MODE, SCALED, NS, 2, ADJ>(in, out, gl, s, tid, m);
 }
+
+// Exponents of a rescaled pass's tiles: the stored values times 2^scale are the tile's, the
+// largest of which lies in [2^(top - 1), 2^top) (kNoTop: no nonzero finite value).
+struct TileExp {
+    int32_t scale, top;
+};
+constexpr int kNoTop = INT32_MIN;
 
 // A pass reads and writes the tensor once in HBM, and each step once in LDS: at 8 steps
 // the two and the multiply-adds take about as long as each other, and two workgroups a CU
@@ -124,8 +170,15 @@ __device__ __forceinline__ void chain_step_nb(const V* in, V* out, const V* gl, 
 // complex64, 1,517 GB step by step, 181 GB in passes): 271.7 ms with k_thin, 99.6 ms;
 // complex128 544 and 225 ms.  Tiles of 2^11 (four workgroups a CU, shorter passes): 103.8
 // and 292 ms.
-template <class V, int MODE>
-__global__ __launch_bounds__(kChainThreads) void k_chain(const V* __restrict__ X, V* __restrict__ C, ChainArgs a) {
+// SCALED: complex64 values may not leave FP32's range between the steps, so a tile whose
+// largest |re|, |im| a step leaves outside [2^-16, 2^16] is scaled by the power of two that
+// brings it into [0.5, 1) (exact; the test is one maximum a value and two ballots a wave, and
+// a tile of gate-sized values never scales).  Step by step every result is scaled, so the
+// values are the same.
+template <class V, int MODE, bool SCALED>
+__global__ __launch_bounds__(kChainThreads) void k_chain(const V* __restrict__ X, V* __restrict__ C, ChainArgs a,
+                                                         TileExp* __restrict__ tile_exp) {
+    static_assert(!SCALED || sizeof(V) == 8, "complex64 values are rescaled");
     constexpr int kTile = (8 << kMaxTileBits) / int(sizeof(V));
     const ChainPlan& p = a.p;
     __shared__ V gl[kMaxLinks][16];
@@ -170,19 +223,55 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(const V* __restrict__ X
             }
     }
     __syncthreads();
+    __shared__ int wave_range[2][kChainThreads / 64];  // of the step before and this one
+    __shared__ float wave_max[kChainThreads / 64];
+    float m = 0.0f;
+    int scale = 0;
+    bool empty = false;  // no nonzero finite value left: nothing to scale from here on
     for (int i = 0; i < p.n_steps; ++i) {
         const ChainStep& s = p.step[i];
+        m = 0.0f;
         switch (s.ns * 4 + s.adj) {
-            case 3: chain_step_nb<V, MODE, 1, -1>(buf, alt, gl[i], s, tid); break;
-            case 4: chain_step_nb<V, MODE, 1, 0>(buf, alt, gl[i], s, tid); break;
-            case 7: chain_step_nb<V, MODE, 2, -1>(buf, alt, gl[i], s, tid); break;
-            case 8: chain_step_nb<V, MODE, 2, 0>(buf, alt, gl[i], s, tid); break;
-            default: chain_step_nb<V, MODE, 2, 1>(buf, alt, gl[i], s, tid); break;
+            case 3: chain_step_nb<V, MODE, SCALED, 1, -1>(buf, alt, gl[i], s, tid, m); break;
+            case 4: chain_step_nb<V, MODE, SCALED, 1, 0>(buf, alt, gl[i], s, tid, m); break;
+            case 7: chain_step_nb<V, MODE, SCALED, 2, -1>(buf, alt, gl[i], s, tid, m); break;
+            case 8: chain_step_nb<V, MODE, SCALED, 2, 0>(buf, alt, gl[i], s, tid, m); break;
+            default: chain_step_nb<V, MODE, SCALED, 2, 1>(buf, alt, gl[i], s, tid, m); break;
         }
         V* const t = buf;
         buf = alt;
         alt = t;
+        if constexpr (SCALED) {
+            const int r = (__any(m >= 0x1p-16f) ? 1 : 0) | (__any(m > 0x1p16f) ? 2 : 0);
+            if ((tid & 63) == 0) wave_range[i & 1][tid >> 6] = r;
+        }
         __syncthreads();
+        if constexpr (SCALED) {
+            int r = 0;
+            for (int w = 0; w < kChainThreads / 64; ++w) r |= wave_range[i & 1][w];
+            if (r != 1 && !empty) {  // the same in every thread
+                const int n = 1 << (s.lb - s.ns + s.nb);
+                const float top = tile_max_finite(buf, n, wave_max);
+                int e = 0;
+                empty = top == 0.0f;
+                if (!empty) (void)frexpf(top, &e);
+                scale += e;
+                for (int k = tid; k < n && e != 0; k += kChainThreads)
+                    buf[k] = V{ldexpf(buf[k].x, -e), ldexpf(buf[k].y, -e)};
+                m = ldexpf(m, -e);
+                __syncthreads();
+            }
+        }
+    }
+    if constexpr (SCALED) {
+        float top = tile_max(m, wave_max);  // of the last step's values
+        if (!(top < INFINITY)) {
+            __syncthreads();
+            top = tile_max_finite(buf, 1 << p.tb_out, wave_max);
+        }
+        int e = 0;
+        (void)frexpf(top, &e);
+        if (tid == 0) tile_exp[id] = TileExp{scale, top > 0.0f ? scale + e : kNoTop};
     }
     int64_t off_t = base_out, off_s[kStepBits];
     for (int b = P; b < hi && b < p.tb_out; ++b)
@@ -199,6 +288,51 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(const V* __restrict__ X
                 if ((q >> k) & 1) off += off_s[k];
             *reinterpret_cast<Pack*>(C + off) = *reinterpret_cast<const Pack*>(buf + (tid << P) + (q << hi));
         }
+}
+
+// Largest top of a rescaled pass's tiles in one workgroup (0 if no tile has one), and C's
+// exponent with X's added.
+constexpr int kTopThreads = 1024;
+__global__ __launch_bounds__(kTopThreads) void k_chain_top(const TileExp* __restrict__ tile_exp, int64_t n,
+                                                           const int32_t* __restrict__ ex, int32_t* __restrict__ ec,
+                                                           int32_t* __restrict__ top) {
+    __shared__ int wave_top[kTopThreads / 64];
+    int t = kNoTop;
+    for (int64_t i = threadIdx.x; i < n; i += kTopThreads) t = max(t, tile_exp[i].top);
+    for (int d = 32; d >= 1; d >>= 1) t = max(t, __shfl_xor(t, d, 64));
+    if ((threadIdx.x & 63) == 0) wave_top[threadIdx.x >> 6] = t;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int w = 1; w < kTopThreads / 64; ++w) t = max(t, wave_top[w]);
+    if (t == kNoTop) t = 0;
+    *top = t;
+    *ec = (ex ? *ex : 0) + t;
+}
+
+// The tiles of C brought to the exponent *top: one workgroup a tile, in k_chain's order.
+__global__ __launch_bounds__(kChainThreads) void k_chain_scale(float2* __restrict__ C, ChainPlan p,
+                                                               const TileExp* __restrict__ tile_exp,
+                                                               const int32_t* __restrict__ top) {
+    const int64_t id = int64_t(blockIdx.x) + int64_t(blockIdx.y) * gridDim.x;
+    const int e = tile_exp[id].scale - *top;
+    if (e == 0) return;
+    int64_t off_t = 0;
+    for (int i = 0; i < p.n_rest; ++i)
+        if ((id >> i) & 1) off_t += int64_t(1) << p.rest_out[i];
+    constexpr int hi = kThreadBits + 1;  // two neighbours a thread, then up to 3 step bits
+    const int tid = threadIdx.x;
+    for (int b = 1; b < hi && b < p.tb_out; ++b)
+        if ((tid >> (b - 1)) & 1) off_t += int64_t(1) << p.out_pos[b];
+    const int n = 1 << p.tb_out;
+    if (2 * tid >= n) return;
+    for (int q = 0; (q << hi) < n; ++q) {
+        int64_t off = off_t;
+        for (int b = hi; b < p.tb_out; ++b)
+            if ((q >> (b - hi)) & 1) off += int64_t(1) << p.out_pos[b];
+        float4* const at = reinterpret_cast<float4*>(C + off);
+        const float4 v = *at;
+        *at = make_float4(ldexpf(v.x, e), ldexpf(v.y, e), ldexpf(v.z, e), ldexpf(v.w, e));
+    }
 }
 
 // Where a bit of the growing tensor comes from: an input position, or a bit that a step added.
@@ -343,14 +477,40 @@ bool plan_chain(int nx, int dl, bool c128, int n, const int32_t* desc, const int
     return true;
 }
 
+// One workgroup a tile.
+dim3 tile_grid(const ChainPlan& p) {
+    const int64_t tiles = int64_t(1) << p.n_rest;
+    const unsigned gx = unsigned(std::min<int64_t>(tiles, 65536));
+    return dim3(gx, unsigned(tiles / gx));
+}
+
 template <class V, int MODE>
 qt_status launch_chain(Ctx* c, const Tensor* X, Tensor* C, const ChainArgs& a) {
-    const int64_t tiles = int64_t(1) << a.p.n_rest;
-    const unsigned gx = unsigned(std::min<int64_t>(tiles, 65536));
-    const unsigned gy = unsigned(tiles / gx);
-    hipLaunchKernelGGL((k_chain<V, MODE>), dim3(gx, gy), dim3(kChainThreads), 0, c->stream,
-                       static_cast<const V*>(X->data), static_cast<V*>(C->data), a);
+    hipLaunchKernelGGL((k_chain<V, MODE, false>), tile_grid(a.p), dim3(kChainThreads), 0, c->stream,
+                       static_cast<const V*>(X->data), static_cast<V*>(C->data), a, static_cast<TileExp*>(nullptr));
     return check_hip(c, hipGetLastError(), "k_chain");
+}
+
+// The same with C scaled: its largest |re|, |im| in [0.5, 1), exponent on the device.
+template <int MODE>
+qt_status launch_chain_scaled(Ctx* c, const Tensor* X, Tensor* C, const ChainArgs& a) {
+    qt_status s = acquire_exponent(c, C);
+    if (s != QT_OK) return s;
+    const int64_t tiles = int64_t(1) << a.p.n_rest;
+    hipError_t e = hipSuccess;
+    auto* const exps = static_cast<TileExp*>(c->pool.alloc(size_t(tiles) * sizeof(TileExp) + 256, &e));
+    if (!exps) return check_hip(c, e, "qt_contract_chain: tile exponents");
+    auto* const top = reinterpret_cast<int32_t*>(exps + tiles);
+    auto* const out = static_cast<float2*>(C->data);
+    hipLaunchKernelGGL((k_chain<float2, MODE, true>), tile_grid(a.p), dim3(kChainThreads), 0, c->stream,
+                       static_cast<const float2*>(X->data), out, a, exps);
+    const int32_t* const ex = X->exp_slot >= 0 ? c->d_exp + X->exp_slot : nullptr;
+    hipLaunchKernelGGL(k_chain_top, dim3(1), dim3(kTopThreads), 0, c->stream, exps, tiles, ex, c->d_exp + C->exp_slot,
+                       top);
+    hipLaunchKernelGGL(k_chain_scale, tile_grid(a.p), dim3(kChainThreads), 0, c->stream, out, a.p, exps, top);
+    s = check_hip(c, hipGetLastError(), "k_chain (rescaled)");
+    c->pool.release(exps);  // later work on this stream may take it
+    return s;
 }
 
 }  // namespace
@@ -407,13 +567,19 @@ qt_status qt_contract_chain(qt_ctx* cx, const qt_tensor* X, int rank_x, int n, c
     qt_status s = qt::check_deadline(ctx, "qt_contract_chain");
     if (s != QT_OK) return s;
     (void)hipSetDevice(ctx->device);
+    if (rescale)
+        switch (form) {
+            case QT_C64_4M: return qt::launch_chain_scaled<qt::MODE_4M>(ctx, &x, &c, a);
+            case QT_C64_3M: return qt::launch_chain_scaled<qt::MODE_3M>(ctx, &x, &c, a);
+            default: return qt::launch_chain_scaled<qt::MODE_BF16X3>(ctx, &x, &c, a);
+        }
     switch (form) {
         case QT_PLAIN_C128: s = qt::launch_chain<double2, qt::MODE_PLAIN>(ctx, &x, &c, a); break;
         case QT_C64_4M: s = qt::launch_chain<float2, qt::MODE_4M>(ctx, &x, &c, a); break;
         case QT_C64_3M: s = qt::launch_chain<float2, qt::MODE_3M>(ctx, &x, &c, a); break;
         default: s = qt::launch_chain<float2, qt::MODE_BF16X3>(ctx, &x, &c, a); break;
     }
-    if (s == QT_OK) s = rescale ? qt::rescale_c64(ctx, &x, &G[0]->impl, &c) : qt::carry_exponent(ctx, &x, &G[0]->impl, &c);
+    if (s == QT_OK) s = qt::carry_exponent(ctx, &x, &G[0]->impl, &c);
     return s;
 }
 

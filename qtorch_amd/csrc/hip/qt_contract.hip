@@ -1658,8 +1658,6 @@ qt_status accumulate_scalar(Ctx* c, const Tensor* t, Tensor* acc) {
     return check_hip(c, hipGetLastError(), "k_accumulate");
 }
 
-namespace {
-
 // The device exponent table (first use) and a slot of it for C.
 qt_status acquire_exponent(Ctx* c, Tensor* C) {
     if (!c->d_exp) {
@@ -1677,6 +1675,8 @@ qt_status acquire_exponent(Ctx* c, Tensor* C) {
     }
     return QT_OK;
 }
+
+namespace {
 
 __global__ void k_carry_exponent(const int32_t* __restrict__ ea, const int32_t* __restrict__ eb,
                                  int32_t* __restrict__ ec) {

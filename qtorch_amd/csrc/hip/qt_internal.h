@@ -132,6 +132,8 @@ qt_status rescale_c64(Ctx* c, const Tensor* A, const Tensor* B, Tensor* C);
 // Reads a tensor's exponent (0 if never rescaled); synchronises.
 qt_status read_exponent(Ctx* c, const Tensor* t, int32_t* e);
 void release_exponent(Ctx* c, Tensor* t);
+// Gives C a slot of the device exponent table (allocated on first use).
+qt_status acquire_exponent(Ctx* c, Tensor* C);
 // exp(C) = exp(A) + exp(B) on the device, for a step without rescaling whose
 // operands carry exponents from earlier rescaled steps.
 qt_status carry_exponent(Ctx* c, const Tensor* A, const Tensor* B, Tensor* C);

@@ -43,6 +43,17 @@ def test_chain_equals_steps(ctx, rank, d, links, prec):
         return qa.Tensor(ctx, r, d, dtype).upload(v)
 
     x = tensor(rank)
+    small, steps, desc, axes = make_links(rng, tensor, rank, links)
+    n = hip.qt_chain_links(rank, d, dtype, len(links), _i32(desc), _i32(axes))
+    assert n >= 2
+    ref = x
+    for g, pairs, free in steps[:n]:
+        ref, _ = qa.contract_pair(ctx, ref, g, pairs, free, prec)
+    assert np.array_equal(run_chain(ctx, x, small[:n], desc, axes, prec).download(), ref.download()), n
+
+
+def make_links(rng, tensor, rank, links):
+    """The small tensors, (tensor, pairs, free) of every step, and the chain's arguments."""
     steps, small, desc, axes, r = [], [], [], [], rank
     for pos, new in links:
         pos = [p % r for p in pos]
@@ -56,15 +67,89 @@ def test_chain_equals_steps(ctx, rank, d, links, prec):
         desc += [len(order), len(pos), r]
         axes += [p for p, _ in pairs] + [q for _, q in pairs]
         axes += [a | qa.QT_FROM_A if from_a else a for from_a, a in free]
-    n = hip.qt_chain_links(rank, d, dtype, len(links), _i32(desc), _i32(axes))
-    assert n >= 2
+    return small, steps, desc, axes
+
+
+def run_chain(ctx, x, small, desc, axes, prec):
+    n = len(small)
+    c = qa.Tensor(ctx, desc[3 * n - 1], x.dim_log2, x.dtype)
+    gs = (ctypes.c_void_p * n)(*[g.handle for g in small])
+    ctx.check(hip.qt_contract_chain(ctx.handle, x.handle, x.rank, n, gs, _i32(desc), _i32(axes), c.handle, prec), "chain")
+    return c
+
+
+EIGHT = [((0, -1), 1), ((-1,), 2), ((5, -1), 1), ((-1,), 2), ((0, -1), 1), ((0,), 2), ((-1,), 1), ((3,), 0)]
+
+
+@pytest.mark.parametrize("prec", [qa.QT_C64_4M, qa.QT_C64_3M, qa.QT_C64_BF16X3])
+@pytest.mark.parametrize("case", ["unit", "1e-6", "1e6", "2^-90", "2^90", "selects", "one tile", "zero", "exponent"])
+def test_rescaled_chain_keeps_the_range_of_steps(ctx, case, prec):
+    """Eight links whose combined scale leaves FP32: the values that rescaling after every
+    step gives.  Scaling by powers of two commutes with every rounding of a step (no value
+    here is subnormal either way), so they are equal."""
+    rng = np.random.default_rng(17)
+    prec |= qa.QT_RESCALE
+    scale = {"1e-6": 1e-6, "1e6": 1e6, "2^-90": 2.0 ** -90, "2^90": 2.0 ** 90}.get(case, 1.0)
+
+    def values(r):
+        return (rng.standard_normal(1 << r) + 1j * rng.standard_normal(1 << r)).astype(np.complex64)
+
+    def small(r):
+        v = values(r) * np.float32(scale)
+        if case == "selects":  # large where the tensor is zero, 1e-6 where it is not
+            v *= np.where(np.arange(1 << r) & 1, np.float32(1e-6), np.float32(1))
+        return qa.Tensor(ctx, r, 1, qa.QT_DTYPE_C64).upload(v)
+
+    v = values(19)
+    links = EIGHT
+    if case == "selects":
+        links = [((0,), 0)] * 8  # the lowest bit summed, nothing added
+        v[(np.arange(v.size) & 255) != 255] = 0  # only bit 1 of every summed wire
+    if case == "one tile":  # most tiles hold no value at all
+        v[: v.size - 1] = 0
+    if case == "zero":
+        v[:] = 0
+    x = qa.Tensor(ctx, 19, 1, qa.QT_DTYPE_C64).upload(v)
+    if case == "exponent":  # X carries one already
+        x, _ = qa.contract_pair(ctx, x, qa.Tensor(ctx, 1, 1, qa.QT_DTYPE_C64).upload(np.array([1e-30, 2e-30])), [],
+                                [(True, i) for i in range(19)] + [(False, 0)], prec)
+        assert x.exponent() < -80
+    gs, steps, desc, axes = make_links(rng, small, x.rank, links)
+    n = hip.qt_chain_links(x.rank, 1, x.dtype, len(links), _i32(desc), _i32(axes))
+    assert n >= 6
     ref = x
     for g, pairs, free in steps[:n]:
         ref, _ = qa.contract_pair(ctx, ref, g, pairs, free, prec)
-    c = qa.Tensor(ctx, desc[3 * n - 1], d, dtype)
-    gs = (ctypes.c_void_p * n)(*[g.handle for g in small[:n]])
-    ctx.check(hip.qt_contract_chain(ctx.handle, x.handle, rank, n, gs, _i32(desc), _i32(axes), c.handle, prec), "chain")
-    assert np.array_equal(c.download(), ref.download()), n
+    c = run_chain(ctx, x, gs[:n], desc, axes, prec)
+    assert c.exponent() == ref.exponent()
+    assert np.array_equal(c.download(), ref.download())
+    assert case == "zero" or 0.5 <= max(np.abs(c.download().view(np.float32))) < 1
+
+
+def test_rescaled_chain_passes_infinities_on(ctx):
+    """An infinite element spoils the outputs it reaches, step by step and in one pass; the
+    others keep their values."""
+    rng = np.random.default_rng(3)
+
+    def tensor(r):
+        v = (rng.standard_normal(1 << r) + 1j * rng.standard_normal(1 << r)).astype(np.complex64)
+        return qa.Tensor(ctx, r, 1, qa.QT_DTYPE_C64).upload(v * np.float32(1e-3))
+
+    v = (rng.standard_normal(1 << 18) + 1j * rng.standard_normal(1 << 18)).astype(np.complex64)
+    v[12345] = np.inf
+    x = qa.Tensor(ctx, 18, 1, qa.QT_DTYPE_C64).upload(v)
+    gs, steps, desc, axes = make_links(rng, tensor, 18, [((0,), 1), ((16,), 1), ((2,), 1)])
+    prec = qa.QT_C64_4M | qa.QT_RESCALE
+    assert hip.qt_chain_links(18, 1, x.dtype, 3, _i32(desc), _i32(axes)) == 3
+    ref = x
+    for g, pairs, free in steps:
+        ref, _ = qa.contract_pair(ctx, ref, g, pairs, free, prec)
+    c = run_chain(ctx, x, gs, desc, axes, prec)
+    got, want = c.download(), ref.download()
+    ok = np.isfinite(want)
+    assert np.array_equal(np.isfinite(got), ok) and not ok.all() and ok.any()
+    assert np.array_equal(np.ldexp(got[ok].view(np.float32).astype(np.float64), c.exponent()),
+                          np.ldexp(want[ok].view(np.float32).astype(np.float64), ref.exponent()))
 
 
 def test_what_does_not_chain(ctx):
