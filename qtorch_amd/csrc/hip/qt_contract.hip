@@ -1759,8 +1759,19 @@ qt_status run_gemm(Ctx* c, const Tensor* A, const Tensor* B, Tensor* C, const Bi
     bool perm_a = !is_identity(src_a, mbits + sb), perm_b = !is_identity(src_b, nbits_n + sb);
     // bf16x3 with whole 128 x 128 x 32 tiles: the permutes write bf16 planes, the lowest
     // three summed bits first (k_gemm_bf16x3).  Each operand then needs scratch of its own
-    // size, also one that is in place, so not with a caller's workspace
-    const bool planes = MODE == MODE_BF16X3 && !ws && mbits >= 7 && nbits_n >= 7 && sb >= 5;
+    // size, also one that is in place, so not with a caller's workspace, and where there is
+    // no room for both, k_gemm_c64 takes the operands as they are
+    bool planes = MODE == MODE_BF16X3 && !ws && mbits >= 7 && nbits_n >= 7 && sb >= 5;
+    if (planes) {
+        hipError_t e = hipSuccess;
+        abuf = c->pool.alloc(A->bytes, &e);
+        if (abuf) bbuf = c->pool.alloc(B->bytes, &e);
+        if (!bbuf) {
+            c->pool.release(abuf);
+            abuf = nullptr;
+            planes = false;
+        }
+    }
     if (planes) {
         auto lowest_first = [&](int* src, int free_bits, const uint8_t* sum) {
             for (int j = free_bits - 1; j >= 0; --j) src[j + 3] = src[j];
@@ -1783,14 +1794,14 @@ qt_status run_gemm(Ctx* c, const Tensor* A, const Tensor* B, Tensor* C, const Bi
     qt_status s = QT_OK;
     if (perm_a) {
         hipError_t e = hipSuccess;
-        abuf = ws ? static_cast<void*>(ws->base) : c->pool.alloc(A->bytes, &e);
+        if (!abuf) abuf = ws ? static_cast<void*>(ws->base) : c->pool.alloc(A->bytes, &e);
         if (!abuf) return check_hip(c, e, "gemm scratch A");
         s = rewrite(A, abuf, mbits + sb, src_a);
         ap = static_cast<const V*>(abuf);
     }
     if (s == QT_OK && perm_b) {
         hipError_t e = hipSuccess;
-        bbuf = ws ? static_cast<void*>(ws->base + ws_b) : c->pool.alloc(B->bytes, &e);
+        if (!bbuf) bbuf = ws ? static_cast<void*>(ws->base + ws_b) : c->pool.alloc(B->bytes, &e);
         if (!bbuf) {
             if (!ws) c->pool.release(abuf);
             return check_hip(c, e, "gemm scratch B");

@@ -8,6 +8,7 @@ import pytest
 
 import qtorch_amd as qa
 from qtorch_amd._native import _i32, hip
+from tests.full_device import full_device
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +48,23 @@ def test_planes(ctx, m, n, k, shuffle):
                                                _i32([x for x, _ in pairs]), _i32([y for _, y in pairs]), m + n, fs,
                                                plain.handle, qa.QT_C64_BF16X3, ctypes.byref(ctypes.c_int64())), "noalloc")
         assert np.array_equal(got, plain.download())
+
+
+@pytest.mark.parametrize("left_mib", [128, 384])
+def test_in_place_product_without_room_for_planes(left_mib):
+    """Operands of 256 MiB in GEMM order on a full card, with room for neither operand's
+    planes or for one's: the product runs on them as they are.  4 output tiles of 64 x 64 or
+    one of 128 x 128, 64 parts of the sum either way, so the results are equal."""
+    ctx = qa.Context(0)
+    m = n = 7
+    k = 18
+    rng = np.random.default_rng(5)
+    v = (rng.standard_normal(1 << 20) + 1j * rng.standard_normal(1 << 20)).astype(np.complex64)
+    a, b = (qa.Tensor(ctx, m + k, 1, qa.QT_DTYPE_C64).upload(np.tile(x, 1 << (m + k - 20))) for x in (v, v[::-1]))
+    pairs = [(m + i, n + i) for i in reversed(range(k))]
+    free = [(True, i) for i in range(m)] + [(False, i) for i in range(n)]
+    want = qa.contract_pair(ctx, a, b, pairs, free, qa.QT_C64_BF16X3)[0].download()
+    ctx.check(hip.qt_ctx_trim(ctx.handle))
+    with full_device(left_mib):
+        got = qa.contract_pair(ctx, a, b, pairs, free, qa.QT_C64_BF16X3)[0].download()
+    assert np.array_equal(got, want)
