@@ -1760,8 +1760,18 @@ qt_status run_gemm(Ctx* c, const Tensor* A, const Tensor* B, Tensor* C, const Bi
     // bf16x3 with whole 128 x 128 x 32 tiles: the permutes write bf16 planes, the lowest
     // three summed bits first (k_gemm_bf16x3).  Each operand then needs scratch of its own
     // size, also one that is in place, so not with a caller's workspace, and where there is
-    // no room for both, k_gemm_c64 takes the operands as they are
-    bool planes = MODE == MODE_BF16X3 && !ws && mbits >= 7 && nbits_n >= 7 && sb >= 5;
+    // no room for both, k_gemm_c64 takes the operands as they are.  An operand in place
+    // pays a pass over it for the planes, so there the product has to be large.  us without
+    // and with planes (2^m x 2^n over 2^k):
+    //   both in place, below 2^30 MACs:  7,7,5 5.3, 15.0;  9,9,8 24, 34;  11,11,7 32, 35
+    //   from there:                      10,10,10 84, 60;  13,13,5 181, 147
+    //   one in place, 2^8 or more terms: 7,7,8 37, 32;     10,10,9 55, 47 (7,7,5 10.3, 14.8;
+    //     10,10,6 17, 21); 32 times the other operand: 12,7,10 50, 54
+    //   both permuted:                   7,7,5 14.3, 14.9; 8,8,10 52, 39; 10,10,12 320, 147
+    const bool one_permuted = perm_a != perm_b;
+    const int excess = perm_a ? nbits_n - mbits : mbits - nbits_n;  // of the one in place, in bits
+    bool planes = MODE == MODE_BF16X3 && !ws && mbits >= 7 && nbits_n >= 7 && sb >= 5 &&
+                  ((perm_a && perm_b) || m.nbits_c + sb >= 30 || (one_permuted && sb >= 8 && excess <= 3));
     if (planes) {
         hipError_t e = hipSuccess;
         abuf = c->pool.alloc(A->bytes, &e);

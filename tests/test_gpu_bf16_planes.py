@@ -1,6 +1,6 @@
 """bf16x3 products on operands rewritten as bf16 planes (k_gemm_bf16x3): the smallest
-shape that takes it, one split over K, uneven sides, and operands already in GEMM order,
-against numpy in complex128 and the path without planes (qt_contract_pair_noalloc)."""
+shape that takes it, one split over K, uneven sides, and one or both operands already in
+GEMM order on either side of the rule, against numpy in complex128 and the path without planes (qt_contract_pair_noalloc)."""
 import ctypes
 
 import numpy as np
@@ -20,7 +20,8 @@ def ctx():
     c.close()
 
 
-@pytest.mark.parametrize("m,n,k,shuffle", [(7, 7, 5, True), (7, 7, 5, False), (8, 7, 6, True), (7, 9, 10, True)])
+@pytest.mark.parametrize("m,n,k,shuffle", [(7, 7, 5, True), (7, 7, 5, False), (8, 7, 6, True), (7, 9, 10, True),
+                                           (8, 7, 8, "A"), (11, 7, 8, "A"), (11, 7, 8, "B"), (9, 8, 13, False)])
 def test_planes(ctx, m, n, k, shuffle):
     rng = np.random.default_rng(100 * m + 10 * n + k)
     a, b = ((rng.standard_normal((1 << k, 1 << f)) + 1j * rng.standard_normal((1 << k, 1 << f))).astype(np.complex64)
@@ -28,8 +29,8 @@ def test_planes(ctx, m, n, k, shuffle):
     ref = (b.astype(np.complex128).T @ a).reshape(-1)  # C[m + M n]
     # wires of A: m free then k summed (axis 0 fastest), moved to the places of a permutation
     tensors, place = [], []
-    for x, f in ((a, m), (b, n)):
-        to = rng.permutation(f + k) if shuffle else np.arange(f + k)  # wire i sits on axis to[i]
+    for name, x, f in (("A", a, m), ("B", b, n)):
+        to = rng.permutation(f + k) if shuffle in (True, name) else np.arange(f + k)  # wire i sits on axis to[i]
         r = f + k
         t = x.reshape([2] * r).transpose([r - 1 - int(np.argwhere(to == ax)[0, 0]) for ax in reversed(range(r))])
         tensors.append(qa.Tensor(ctx, r, 1, qa.QT_DTYPE_C64).upload(np.ascontiguousarray(t)))
