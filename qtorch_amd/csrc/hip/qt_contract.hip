@@ -1079,8 +1079,9 @@ void order_summed_bits(BitMap& m) {
     std::memcpy(m.s_b, sb, size_t(n));
 }
 
+// *no_room: nothing was queued, the partial sums found no device memory.
 template <class V, int MODE>
-qt_status run_reduce(Ctx* c, const V* A, const V* B, V* C, const BitMap& m0, const Workspace* ws) {
+qt_status run_reduce(Ctx* c, const V* A, const V* B, V* C, const BitMap& m0, const Workspace* ws, bool* no_room) {
     BitMap m = m0;
     order_summed_bits(m);
     const int64_t nC = int64_t(1) << m.nbits_c;
@@ -1141,8 +1142,12 @@ qt_status run_reduce(Ctx* c, const V* A, const V* B, V* C, const BitMap& m0, con
                     c->partials = nullptr;
                     c->partials_bytes = 0;
                 }
-                qt_status s = check_hip(c, hipMalloc(&c->partials, need), "partials");
-                if (s != QT_OK) return s;
+                if (hipMalloc(&c->partials, need) != hipSuccess) {
+                    (void)hipGetLastError();
+                    c->partials = nullptr;
+                    *no_room = true;
+                    return QT_OOM;
+                }
                 c->partials_bytes = need;
             }
             part = static_cast<V*>(c->partials);
@@ -1959,7 +1964,11 @@ qt_status dispatch_small(Ctx* c, const Tensor* A, const Tensor* B, Tensor* C, co
     const V* a = static_cast<const V*>(A->data);
     const V* b = static_cast<const V*>(B->data);
     V* cc = static_cast<V*>(C->data);
-    if (reduce_shape(m, ws)) return run_reduce<V, MODE>(c, a, b, cc, m, ws);
+    if (reduce_shape(m, ws)) {
+        bool no_room = false;  // then as sums too short to split, which need no scratch
+        const qt_status s = run_reduce<V, MODE>(c, a, b, cc, m, ws, &no_room);
+        if (!no_room) return s;
+    }
     if (skinny_shape(m, split, mbits)) return run_skinny<V, MODE>(c, a, b, cc, m, mbits);
     return run_direct<V, MODE>(c, a, b, cc, m);
 }

@@ -6,16 +6,19 @@ import torch
 
 @contextlib.contextmanager
 def full_device(left_mib):
-    """Holds device memory so that no more than left_mib MiB (a multiple of 64, to within
-    the driver's granules) can be allocated."""
+    """Holds device memory so that less than left_mib + 12 MiB (left_mib a multiple of 64)
+    can be allocated."""
     torch.cuda.empty_cache()
-    step = 64 << 20
-    held = [torch.empty(max(torch.cuda.mem_get_info()[0] - (2 << 30), step), dtype=torch.uint8, device="cuda")]
-    while True:  # the driver gives more than it reports free
-        try:
-            held.append(torch.empty(step, dtype=torch.uint8, device="cuda"))
-        except torch.OutOfMemoryError:
-            break
+    most = 64 << 20
+    held = [torch.empty(max(torch.cuda.mem_get_info()[0] - (2 << 30), most), dtype=torch.uint8, device="cuda")]
+    for step in (most, 12 << 20):  # the driver gives more than it reports free
+        if step < most and left_mib > 0:
+            continue
+        while True:
+            try:
+                held.append(torch.empty(step, dtype=torch.uint8, device="cuda"))
+            except torch.OutOfMemoryError:
+                break
     del held[len(held) - left_mib // 64:]
     torch.cuda.empty_cache()
     try:

@@ -6,6 +6,8 @@ import numpy as np
 import pytest
 
 import qtorch_amd as qa
+from qtorch_amd._native import _i32, hip
+from tests.full_device import full_device
 
 pytestmark = pytest.mark.gpu
 
@@ -53,3 +55,26 @@ def test_long_sums(ctx, fa, fb, k, d, prec, tol):
         # sums of 2^(d k) products of unit variance: rounding of about sqrt(2^(d k)) terms
         bound = 1e-13 if c128 else tol
         assert np.abs(got - ref).max() <= bound * np.sqrt(1 << (d * k)) * max(np.abs(ref).max(), 1.0)
+
+
+def test_long_sum_without_room_for_partial_sums():
+    """16 MiB of partial sums on a card without them: the sum runs one output a lane."""
+    ctx = qa.Context(0)
+    rng = np.random.default_rng(8)
+    v = (rng.standard_normal(1 << 20) + 1j * rng.standard_normal(1 << 20)).astype(np.complex64)
+    k, fa, fb = 20, 6, 7
+    a, b = (qa.Tensor(ctx, f + k, 1, qa.QT_DTYPE_C64).upload(np.tile(x, 1 << f)) for f, x in ((fa, v), (fb, v[::-1])))
+    pairs = [(i, i) for i in range(k)]  # every row of A equals v, every row of B its reverse
+    free = [(i % 2 == 1, k + i // 2) for i in range(2 * fa)] + [(False, k + fa)]  # B and A in turn: no GEMM
+    c = qa.Tensor(ctx, fa + fb, 1, qa.QT_DTYPE_C64)
+    fs = _i32([(ax | qa.QT_FROM_A) if from_a else ax for from_a, ax in free])
+    px = _i32([x for x, _ in pairs])
+    ctx.check(hip.qt_ctx_trim(ctx.handle))
+    with full_device(0):
+        ctx.check(hip.qt_contract_pair(ctx.handle, a.handle, fa + k, b.handle, fb + k, k, px, px, fa + fb, fs, c.handle,
+                                       qa.QT_C64_4M, None))
+        ctx.sync()
+    got = c.download()
+    ref = np.dot(v.astype(np.complex128), v[::-1])
+    # 2^21 roundings of partial sums of up to about 2^10.5, independent: 2^-24 2^10.5 2^10.5, four times over
+    assert np.abs(got - ref).max() <= 0.5
