@@ -791,6 +791,42 @@ qt_status order_instances(qt_batch* b) {
     return s;
 }
 
+// Workgroups per CU of a shape the caller did not choose.  Workgroup executors wait on memory
+// most of the time, four to a CU hide some of it: 1,920 complex64 networks of 0.01 to 10
+// million MACs, intermediates in device memory, take 1,465 / 928 / 843 us at 1 / 2 / 4 (two
+// where that keeps the intermediates in LDS).
+int default_wgs(const qt_batch* b) {
+    const size_t per_exec = size_t(b->scratch_elems) * elem_size(b->precision);
+    return b->lanes == 256 && per_exec > 32 * 1024 && per_exec <= 64 * 1024 ? 2 : 4;
+}
+
+// LDS unless it does not fit or would hold fewer workgroups per CU than asked for (then the
+// intermediates go through L1/L2); an explicit placement wins.
+qt_status place_scratch(qt_batch* b) {
+    Ctx* c = b->ctx;
+    const size_t es = elem_size(b->precision);
+    const int kExec = execs_per_wg(b->lanes);
+    const size_t stage = b->stage_leaves ? (size_t(kExec) * size_t(b->pstage) + size_t(b->cstage)) * es : 0;
+    const size_t per_wg = size_t(kExec) * size_t(b->slot_stride) * es;
+    const size_t wgs_on_cu = size_t(b->wgs_per_cu) * (b->lanes >= 64 ? 1 : 4);
+    const size_t lds_need = per_wg + stage, lds_cap = 160 * 1024, most = size_t(4) << 30;
+    const int place = b->scratch_place & 3;
+    if (place == QT_SCRATCH_LDS && lds_need > 64 * 1024)
+        return set_error(c, QT_INVALID_INPUT, "batch: the executors' scratch does not fit a workgroup's LDS");
+    b->use_global_scratch = place == QT_SCRATCH_GLOBAL ||
+                            (place == QT_SCRATCH_AUTO && (lds_need * wgs_on_cu > lds_cap || lds_need > 64 * 1024));
+    if (!b->use_global_scratch) return QT_OK;
+    const size_t need = size_t(grid_wgs(b)) * per_wg;
+    if (need > most) return set_error(c, QT_OOM, "batch: scratch of this executor shape exceeds 4 GiB");
+    if (need <= b->global_scratch_bytes) return QT_OK;
+    batch_free(c, b->d_global_scratch);
+    b->d_global_scratch = nullptr;
+    b->global_scratch_bytes = 0;
+    qt_status s = check_hip(c, batch_malloc(c, &b->d_global_scratch, need), "batch global scratch");
+    if (s == QT_OK) b->global_scratch_bytes = need;
+    return s;
+}
+
 qt_status configure_scratch(qt_batch* b) {
     Ctx* c = b->ctx;
     b->shape_ok = false;  // set once the arrays below match the executor shape
@@ -801,19 +837,19 @@ qt_status configure_scratch(qt_batch* b) {
     b->slot_stride = b->lanes < 64 ? b->scratch_elems + 1 : b->scratch_elems;
     // leaf stages of lane-grouped waves (LDS in either placement)
     b->stage_leaves = b->lanes < 64 && (b->scratch_place & QT_SCRATCH_STAGE_LEAVES);
-    const size_t stage = b->stage_leaves ? (size_t(kExec) * size_t(b->pstage) + size_t(b->cstage)) * es : 0;
-    const size_t lds_need = size_t(kExec) * size_t(b->slot_stride) * es + stage;
-    const size_t lds_cap = 160 * 1024;
-    const size_t wgs_on_cu = size_t(b->wgs_per_cu) * (b->lanes >= 64 ? 1 : 4);
-    if (stage > 64 * 1024)
+    if (b->stage_leaves && (size_t(kExec) * size_t(b->pstage) + size_t(b->cstage)) * es > 64 * 1024)
         return set_error(c, QT_INVALID_INPUT, "batch: the leaf stages do not fit a workgroup's LDS");
-    const int place = b->scratch_place & 3;
-    if (place == QT_SCRATCH_LDS && lds_need > 64 * 1024)
-        return set_error(c, QT_INVALID_INPUT, "batch: the executors' scratch does not fit a workgroup's LDS");
-    // LDS unless it does not fit or would hold fewer workgroups per CU than asked for
-    // (then the intermediates go through L1/L2); an explicit placement wins
-    b->use_global_scratch = place == QT_SCRATCH_GLOBAL ||
-                            (place == QT_SCRATCH_AUTO && (lds_need * wgs_on_cu > lds_cap || lds_need > 64 * 1024));
+    // a default shape takes fewer workgroups where its scratch passes 4 GiB or finds no
+    // room; the programs may have grown since it was chosen
+    if (b->default_shape) b->wgs_per_cu = default_wgs(b);
+    const std::string err = c->err;
+    qt_status s = place_scratch(b);
+    while (s == QT_OOM && b->default_shape && b->wgs_per_cu > 1) {
+        b->wgs_per_cu /= 2;
+        s = place_scratch(b);
+        if (s == QT_OK) c->err = err;
+    }
+    if (s != QT_OK) return s;
     // chunks of consecutive instances of one program, at most one per instance slot
     if (b->lanes < 64) {
         const int W = 64 / b->lanes;
@@ -824,27 +860,12 @@ qt_status configure_scratch(qt_batch* b) {
             ch.push_back(int2{i, j - i});
             i = j;
         }
-        qt_status s = dev_put(c, &b->d_chunks, &b->cap_chunks, ch.data(), ch.size());
-        if (s != QT_OK) return s;
+        s = dev_put(c, &b->d_chunks, &b->cap_chunks, ch.data(), ch.size());
         b->n_chunks = int(ch.size());
+    } else {
+        s = order_instances(b);
     }
-    else {
-        qt_status s = order_instances(b);
-        if (s != QT_OK) return s;
-    }
-    if (b->use_global_scratch) {
-        const size_t need = size_t(grid_wgs(b)) * size_t(kExec) * size_t(b->slot_stride) * es;
-        if (need > (size_t(4) << 30))
-            return set_error(c, QT_OOM, "batch: scratch of this executor shape exceeds 4 GiB");
-        if (need > b->global_scratch_bytes) {
-            batch_free(c, b->d_global_scratch);
-            b->d_global_scratch = nullptr;
-            b->global_scratch_bytes = 0;
-            qt_status s = check_hip(c, batch_malloc(c, &b->d_global_scratch, need), "batch global scratch");
-            if (s != QT_OK) return s;
-            b->global_scratch_bytes = need;
-        }
-    }
+    if (s != QT_OK) return s;
     if (b->graph_exec) {
         (void)hipGraphExecDestroy(b->graph_exec);
         b->graph_exec = nullptr;
@@ -1319,14 +1340,6 @@ qt_status qt_batch_create(qt_ctx* cx, int n_programs, qt_program* const* progs, 
         // default executor shape from the scratch footprint (the autotuner may refine it)
         const size_t per_exec = size_t(b->scratch_elems) * qt::elem_size(precision);
         b->lanes = per_exec * 4 <= 16 * 1024 ? 64 : 256;
-        // workgroup executors wait on memory most of the time, four to a CU hide some of
-        // it: 1,920 complex64 networks of 0.01 to 10 million MACs, intermediates in device
-        // memory, take 1,465 / 928 / 843 us at 1 / 2 / 4 (two where that keeps the
-        // intermediates in LDS; fewer where the scratch area would pass 4 GiB)
-        b->wgs_per_cu = per_exec > 32 * 1024 && per_exec <= 64 * 1024 ? 2 : 4;
-        while (b->lanes == 256 && b->wgs_per_cu > 1 &&
-               per_exec * size_t(b->n_cus) * size_t(b->wgs_per_cu) > (size_t(4) << 30))
-            b->wgs_per_cu /= 2;
         s = qt::configure_scratch(b.get());
     }
     if (s != QT_OK) {
@@ -1501,6 +1514,8 @@ qt_status qt_batch_config_ex(qt_batch* b, int lanes, int wgs_per_cu, int scratch
     std::lock_guard<std::recursive_mutex> g(b->ctx->mu);
     qt::drop_specialised(b);  // an explicit table-executor shape replaces generated code
     const int l0 = b->lanes, w0 = b->wgs_per_cu, s0 = b->scratch_place;
+    const bool d0 = b->default_shape;
+    b->default_shape = false;
     b->lanes = lanes;
     b->wgs_per_cu = wgs_per_cu;
     b->scratch_place = scratch;
@@ -1509,6 +1524,7 @@ qt_status qt_batch_config_ex(qt_batch* b, int lanes, int wgs_per_cu, int scratch
         b->lanes = l0;
         b->wgs_per_cu = w0;
         b->scratch_place = s0;
+        b->default_shape = d0;
         (void)qt::configure_scratch(b);
     }
     return s;
