@@ -816,8 +816,10 @@ qt_status place_scratch(qt_batch* b) {
     b->use_global_scratch = place == QT_SCRATCH_GLOBAL ||
                             (place == QT_SCRATCH_AUTO && (lds_need * wgs_on_cu > lds_cap || lds_need > 64 * 1024));
     if (!b->use_global_scratch) return QT_OK;
-    const size_t need = size_t(grid_wgs(b)) * per_wg;
-    if (need > most) return set_error(c, QT_OOM, "batch: scratch of this executor shape exceeds 4 GiB");
+    // a chosen shape stands or falls by its full grid, however few the instances of the moment
+    const size_t full = size_t(b->n_cus) * wgs_on_cu * per_wg;
+    if (full > most) return set_error(c, QT_OOM, "batch: scratch of this executor shape exceeds 4 GiB");
+    const size_t need = b->default_shape ? size_t(grid_wgs(b)) * per_wg : full;
     if (need <= b->global_scratch_bytes) return QT_OK;
     batch_free(c, b->d_global_scratch);
     b->d_global_scratch = nullptr;

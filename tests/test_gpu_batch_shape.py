@@ -90,3 +90,17 @@ def test_programs_added_to_a_default_shape(ctx):
     # 16 sums of 2^8 terms, each rounding relative to the terms' norms (about 2 each here)
     assert np.abs(got[1:] - ref).max() <= 1e-12 * max(abs(ref), 1)
     b.close()
+
+
+def test_chosen_shape_beyond_the_bound_is_refused(ctx):
+    """However few the instances; the shape before it stays."""
+    b = Batch(ctx, [large_program(ctx)], qa.QT_PLAIN_C128)
+    b.set(pool(), [0])
+    first = b.run()
+    before = b.shape()
+    assert b.config(256, 4) == QT_OOM and b.config(256, 16) == QT_OOM
+    assert b.shape() == before
+    assert np.array_equal(b.run(), first)
+    assert b.config(256, 1) == QT_OK
+    assert np.array_equal(b.run(), first)
+    b.close()
