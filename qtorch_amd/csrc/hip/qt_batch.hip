@@ -101,7 +101,8 @@ __device__ __forceinline__ void exec_sync() {
     }
 }
 
-template <class V, int MODE, int LANES, class PA, class PB>
+// LARGE: sums of 16 or more keep 16 operand pairs in flight (64 to 128 registers).
+template <class V, int MODE, int LANES, bool LARGE, class PA, class PB>
 __device__ __forceinline__ void run_step(PA A, PB B, V* C, const uint32_t* __restrict__ fc,
                                          const uint32_t* __restrict__ gs, int nC, int K, int lane,
                                          double2* out_final, V* stage = nullptr) {
@@ -191,7 +192,7 @@ __device__ __forceinline__ void run_step(PA A, PB B, V* C, const uint32_t* __res
         const auto pa = A + int(f & 0xffffu);
         const auto pb = B + int(f >> 16);
         Acc<V, MODE> acc;
-        if ((K & 15) == 0) {
+        if (LARGE && (K & 15) == 0) {
             // 16 operand pairs in flight
             for (int s = 0; s < K; s += 16) {
                 V x[16], y[16];
@@ -377,11 +378,18 @@ inline int32_t mfma_flags(int mbits, int nbits, int k_bits) {
     return ok ? kStepMfma | (mbits << 8) : 0;
 }
 
-template <class V, int MODE, int LANES, class PA, class PB>
+// Steps that the registers of k_batch's LARGE instance are for (two to three waves a SIMD
+// instead of four to eight): a batch without any runs the other one.
+inline bool large_step(const StepDesc& st) {
+    return (st.flags & kStepMfma) || (st.k_bits >= 4 && st.nc_bits + st.k_bits >= 12) ||
+           (st.k_bits >= 8 && st.nc_bits == 0);
+}
+
+template <class V, int MODE, int LANES, bool LARGE, class PA, class PB>
 __device__ __forceinline__ void run_step_any(PA A, PB B, V* C, const uint32_t* __restrict__ fc,
                                              const uint32_t* __restrict__ gs, const StepDesc& st, int lane,
                                              double2* out_final, V* stage) {
-    if constexpr (LANES >= 64 && MODE != QT_C64_BF16X3) {
+    if constexpr (LARGE && MODE != QT_C64_BF16X3) {
         if (st.flags & kStepMfma) {
             const int mb = (st.flags >> 8) & 0xff, nb = st.nc_bits - mb, K = 1 << st.k_bits;
             constexpr int kWaves = LANES / 64;
@@ -400,12 +408,12 @@ __device__ __forceinline__ void run_step_any(PA A, PB B, V* C, const uint32_t* _
             return;
         }
     }
-    run_step<V, MODE, LANES>(A, B, C, fc, gs, 1 << st.nc_bits, 1 << st.k_bits, lane, out_final, stage);
+    run_step<V, MODE, LANES, LARGE>(A, B, C, fc, gs, 1 << st.nc_bits, 1 << st.k_bits, lane, out_final, stage);
 }
 
 // With TOUT, every instance's last step writes its whole result (a tensor, or a
 // scalar) to the instance's output tensor tout[i] instead of the FP64 value array.
-template <class V, int MODE, int LANES, bool GLOBAL_SCRATCH, bool TOUT>
+template <class V, int MODE, int LANES, bool GLOBAL_SCRATCH, bool TOUT, bool LARGE>
 __global__ __launch_bounds__(kWg) void k_batch(const ProgHdr* __restrict__ progs, const StepDesc* __restrict__ steps,
                                                const uint32_t* __restrict__ tabs,
                                                const int64_t* __restrict__ leaf_refs, const V* __restrict__ pool,
@@ -420,11 +428,13 @@ __global__ __launch_bounds__(kWg) void k_batch(const ProgHdr* __restrict__ progs
     const int lane = threadIdx.x % LANES;
     V* mem;
     V* stage = nullptr;  // of the executor's (first) wave, where intermediates are in device memory
-    if constexpr (GLOBAL_SCRATCH) {
+    if constexpr (GLOBAL_SCRATCH && LARGE) {
         __shared__ V stages[kExec][128];
         stage = stages[ex];
+    }
+    if constexpr (GLOBAL_SCRATCH)
         mem = gscratch + (int64_t(blockIdx.x) * kExec + ex) * scratch_elems;
-    } else
+    else
         mem = reinterpret_cast<V*>(lds_raw) + ex * scratch_elems;
     while (true) {
         int i;
@@ -465,13 +475,13 @@ __global__ __launch_bounds__(kWg) void k_batch(const ProgHdr* __restrict__ progs
                 return pool + off;
             };
             if (st.a < 0 && st.b < 0)
-                run_step_any<V, MODE, LANES>(leaf(st.a), leaf(st.b), C, fc, gs, st, lane, fin, stage);
+                run_step_any<V, MODE, LANES, LARGE>(leaf(st.a), leaf(st.b), C, fc, gs, st, lane, fin, stage);
             else if (st.a < 0)
-                run_step_any<V, MODE, LANES>(leaf(st.a), (const V*)(mem + st.b), C, fc, gs, st, lane, fin, stage);
+                run_step_any<V, MODE, LANES, LARGE>(leaf(st.a), (const V*)(mem + st.b), C, fc, gs, st, lane, fin, stage);
             else if (st.b < 0)
-                run_step_any<V, MODE, LANES>((const V*)(mem + st.a), leaf(st.b), C, fc, gs, st, lane, fin, stage);
+                run_step_any<V, MODE, LANES, LARGE>((const V*)(mem + st.a), leaf(st.b), C, fc, gs, st, lane, fin, stage);
             else
-                run_step_any<V, MODE, LANES>((const V*)(mem + st.a), (const V*)(mem + st.b), C, fc, gs, st, lane, fin, stage);
+                run_step_any<V, MODE, LANES, LARGE>((const V*)(mem + st.a), (const V*)(mem + st.b), C, fc, gs, st, lane, fin, stage);
             exec_sync<LANES, GLOBAL_SCRATCH>();
         }
     }
@@ -550,13 +560,13 @@ __global__ __launch_bounds__(64) void k_batch_grouped(const ProgHdr* __restrict_
             };
             if (active) {
                 if (st.a < 0 && st.b < 0)
-                    run_step<V, MODE, G>(leaf(st.a), leaf(st.b), C, fc, gs, nC, K, gl, fin);
+                    run_step<V, MODE, G, true>(leaf(st.a), leaf(st.b), C, fc, gs, nC, K, gl, fin);
                 else if (st.a < 0)
-                    run_step<V, MODE, G>(leaf(st.a), (const V*)(mem + st.b), C, fc, gs, nC, K, gl, fin);
+                    run_step<V, MODE, G, true>(leaf(st.a), (const V*)(mem + st.b), C, fc, gs, nC, K, gl, fin);
                 else if (st.b < 0)
-                    run_step<V, MODE, G>((const V*)(mem + st.a), leaf(st.b), C, fc, gs, nC, K, gl, fin);
+                    run_step<V, MODE, G, true>((const V*)(mem + st.a), leaf(st.b), C, fc, gs, nC, K, gl, fin);
                 else
-                    run_step<V, MODE, G>((const V*)(mem + st.a), (const V*)(mem + st.b), C, fc, gs, nC, K, gl, fin);
+                    run_step<V, MODE, G, true>((const V*)(mem + st.a), (const V*)(mem + st.b), C, fc, gs, nC, K, gl, fin);
             }
             exec_sync<64, GLOBAL_SCRATCH>();
         }
@@ -700,7 +710,13 @@ qt_status launch_batch_t(qt_batch* b) {
     auto d_out = reinterpret_cast<double2*>(b->d_out);
     V* const* tout = reinterpret_cast<V* const*>(b->d_tout);
 #define QT_LAUNCH_T(L, G, T)                                                                                       \
-    hipLaunchKernelGGL((k_batch<V, MODE, L, G, T>), dim3(grid), dim3(kWg), lds, c->stream, b->d_progs, b->d_steps, \
+    if (b->large_steps) {                                                                                          \
+        QT_LAUNCH_M(L, G, T, true);                                                                                \
+    } else {                                                                                                       \
+        QT_LAUNCH_M(L, G, T, false);                                                                               \
+    }
+#define QT_LAUNCH_M(L, G, T, M)                                                                                    \
+    hipLaunchKernelGGL((k_batch<V, MODE, L, G, T, M>), dim3(grid), dim3(kWg), lds, c->stream, b->d_progs, b->d_steps, \
                        b->d_tabs, b->d_leaf_refs, pool, b->d_inst, b->n_inst, b->d_order, b->d_counter, d_out,    \
                        gs, b->scratch_elems, tout)
 #define QT_LAUNCH(L, G)              \
@@ -724,6 +740,7 @@ qt_status launch_batch_t(qt_batch* b) {
     }
 #undef QT_LAUNCH
 #undef QT_LAUNCH_T
+#undef QT_LAUNCH_M
     return check_hip(c, hipGetLastError(), "k_batch");
 }
 
@@ -791,13 +808,17 @@ qt_status order_instances(qt_batch* b) {
     return s;
 }
 
-// Workgroups per CU of a shape the caller did not choose.  Workgroup executors wait on memory
-// most of the time, four to a CU hide some of it: 1,920 complex64 networks of 0.01 to 10
-// million MACs, intermediates in device memory, take 1,465 / 928 / 843 us at 1 / 2 / 4 (two
-// where that keeps the intermediates in LDS).
+// Workgroups per CU of a shape the caller did not choose: up to four, since executors wait on
+// memory most of the time (1,920 complex64 networks of 0.01 to 10 million MACs, intermediates
+// in device memory: 1,465 / 928 / 843 us at 1 / 2 / 4), two where that keeps the intermediates
+// in LDS.  In device memory no more than run at once, as each has its scratch: k_batch's LARGE
+// instance holds 245 registers in complex128, 180 in 3M (two waves a SIMD), 147 in 4M (three).
 int default_wgs(const qt_batch* b) {
     const size_t per_exec = size_t(b->scratch_elems) * elem_size(b->precision);
-    return b->lanes == 256 && per_exec > 32 * 1024 && per_exec <= 64 * 1024 ? 2 : 4;
+    if (b->lanes != 256 || per_exec <= 32 * 1024) return 4;
+    if (per_exec <= 64 * 1024) return 2;
+    if (!b->large_steps || b->precision == QT_C64_BF16X3) return 4;
+    return b->precision == QT_C64_4M ? 3 : 2;
 }
 
 // LDS unless it does not fit or would hold fewer workgroups per CU than asked for (then the
@@ -847,7 +868,7 @@ qt_status configure_scratch(qt_batch* b) {
     const std::string err = c->err;
     qt_status s = place_scratch(b);
     while (s == QT_OOM && b->default_shape && b->wgs_per_cu > 1) {
-        b->wgs_per_cu /= 2;
+        --b->wgs_per_cu;
         s = place_scratch(b);
         if (s == QT_OK) c->err = err;
     }
@@ -905,6 +926,7 @@ qt_status append_programs(qt_batch* b, int n, qt_program* const* progs, const in
         const int32_t tab0 = int32_t(b->h_tabs.size());
         for (auto st : p->steps) {
             st.tab += tab0;
+            b->large_steps = b->large_steps || large_step(st);
             b->h_steps.push_back(st);
         }
         b->h_tabs.insert(b->h_tabs.end(), p->tables.begin(), p->tables.end());

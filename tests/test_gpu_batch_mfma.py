@@ -8,6 +8,7 @@ import pytest
 
 import qtorch_amd as qa
 from qtorch_amd import workloads as wl
+from tests.programs import Batch, Program
 
 GOLDEN_DIR = os.path.join(os.path.dirname(__file__), "golden")
 pytestmark = pytest.mark.gpu
@@ -53,3 +54,29 @@ def test_grid_networks(ctx, prec, dim_log2, rows, cols, depth):
                     dim_log2=dim_log2)
     _same_bits(b)
     b.close()
+
+
+@pytest.mark.parametrize("prec", [qa.QT_PLAIN_C128, qa.QT_C64_4M, qa.QT_C64_3M, qa.QT_C64_BF16X3])
+def test_small_programs_beside_large_ones(ctx, prec):
+    """A batch without large steps runs the kernel that has no registers for them; the same
+    program in a batch with one, the other kernel: the same bits."""
+    small = Program(ctx, 1, [4, 4, 4, 3, 1], [0, 16, 32, 48, 56], [
+        (0, 1, 4, 4, [(3, 0), (2, 2)], [(True, 0), (False, 1), (True, 1), (False, 3)]),
+        (2, 3, 4, 3, [(0, 1), (3, 0)], [(False, 2), (True, 1), (True, 2)]),
+        (5, 6, 4, 3, [(0, 0), (2, 2), (3, 1)], [(True, 1)]),
+        (7, 4, 1, 1, [(0, 0)], [])])
+    large = Program(ctx, 1, [9, 9, 8], [0, 64, 128], [
+        (0, 1, 9, 9, [(4 + i, 4 + i) for i in range(5)], [(True, i) for i in range(4)] + [(False, i) for i in range(4)]),
+        (3, 2, 8, 8, [(i, i) for i in range(8)], [])])
+    rng = np.random.default_rng(10)
+    pool = rng.standard_normal(1024) + 1j * rng.standard_normal(1024)
+    alone, beside = Batch(ctx, [small], prec), Batch(ctx, [large, small], prec)
+    alone.set(pool, [0, 0])
+    beside.set(pool, [1, 0, 1])
+    for lanes, place in ((64, qa.QT_SCRATCH_LDS), (64, qa.QT_SCRATCH_GLOBAL), (256, qa.QT_SCRATCH_LDS),
+                         (256, qa.QT_SCRATCH_GLOBAL)):
+        assert alone.config(lanes, 2, place) == 0 and beside.config(lanes, 2, place) == 0
+        x, y = alone.run(), beside.run()
+        assert np.array_equal(x, y[[0, 2]]) and x[0] != 0 and y[1] != 0, (lanes, place)
+    alone.close()
+    beside.close()
