@@ -56,6 +56,83 @@ def test_grid_networks(ctx, prec, dim_log2, rows, cols, depth):
     b.close()
 
 
+def _variant(mb, nb, kb):
+    """The block of 16 x 16 tiles a wave takes for 2^mb x 2^nb outputs over 2^kb, None for
+    vector steps."""
+    if mb < 4 or nb < 4 or kb < 2 or mb + nb + kb < 12:
+        return None
+    blocks = mb + nb - 8
+    if kb >= 3 and blocks >= 4 and mb >= 5 and nb >= 5:
+        return 2, 2
+    if kb >= 3 and blocks >= 3:
+        return (1, 2) if nb >= 5 else (2, 1)
+    return 1, 1
+
+
+SHAPES = {
+    (1, 1): [(4, 6, 2), (6, 4, 2), (5, 5, 2), (4, 5, 3), (4, 4, 4), (4, 4, 5), (5, 4, 6), (4, 4, 8)],
+    (1, 2): [(4, 7, 3), (5, 6, 4), (4, 8, 4), (4, 7, 5), (4, 8, 6)],
+    (2, 1): [(7, 4, 3), (8, 4, 4), (7, 4, 5), (8, 4, 6)],
+    (2, 2): [(6, 6, 3), (6, 6, 4), (5, 7, 5), (7, 5, 5), (6, 6, 6), (8, 8, 3)],
+    None: [(3, 6, 4), (6, 3, 4), (5, 5, 1), (4, 4, 3)],
+}
+
+
+@pytest.mark.parametrize("prec", [qa.QT_PLAIN_C128, qa.QT_C64_4M, qa.QT_C64_3M])
+@pytest.mark.parametrize("variant", SHAPES)
+def test_every_block_shape(ctx, prec, variant):
+    """A step with C's low axes from A and its high ones from B against the same sums with an
+    axis of A moved to the top of C, which the matrix cores do not take: operands that are
+    leaves, intermediates in LDS and in device memory, tensor results, 64 and 256 lanes."""
+    c128 = prec == qa.QT_PLAIN_C128
+    dtype = qa.QT_DTYPE_C128 if c128 else qa.QT_DTYPE_C64
+    rng = np.random.default_rng(9)
+    pool = rng.standard_normal(1 << 18) + 1j * rng.standard_normal(1 << 18)
+    placed = set()
+    for mb, nb, kb in SHAPES[variant]:
+        assert _variant(mb, nb, kb) == variant
+        pairs = [(mb + i, nb + kb - 1 - i) for i in range(kb)]
+        low, high = [(True, i) for i in range(mb)], [(False, i) for i in range(nb)]
+        if variant is None or kb == 2:  # B's summed axes first, too
+            pairs, high = [(mb + i, i) for i in range(kb)], [(False, kb + i) for i in range(nb)]
+        for a_made, b_made in ((False, False), (True, False), (False, True), (True, True)):
+            # an operand that is made: the outer product of two leaves
+            ranks, offsets, steps, at = [], [], [], {}
+            for name, r, made in (("a", mb + kb, a_made), ("b", nb + kb, b_made)):
+                at[name] = len(ranks)
+                for part in ((r // 2, r - r // 2) if made else (r,)):
+                    offsets.append(offsets[-1] + (1 << ranks[-1]) if ranks else 0)
+                    ranks.append(part)
+            ids = {}
+            for name, r, made in (("a", mb + kb, a_made), ("b", nb + kb, b_made)):
+                i = at[name]
+                ids[name] = i
+                if made:
+                    outer = [(True, k) for k in range(ranks[i])] + [(False, k) for k in range(ranks[i + 1])]
+                    ids[name] = len(ranks) + len(steps)
+                    steps.append((i, i + 1, ranks[i], ranks[i + 1], [], outer))
+            last = (ids["a"], ids["b"], mb + kb, nb + kb, pairs)
+            split = Program(ctx, 1, ranks, offsets, steps + [last + (low + high,)])
+            moved = Program(ctx, 1, ranks, offsets, steps + [last + (low[:-1] + high + low[-1:],)])
+            batch = Batch(ctx, [split, moved], prec)
+            outs = [qa.Tensor(ctx, mb + nb, 1, dtype) for _ in range(2)]
+            batch.set(pool, [0, 1])
+            batch.set_outputs(outs)
+            for lanes in (64, 256):
+                for place in (qa.QT_SCRATCH_LDS, qa.QT_SCRATCH_GLOBAL):
+                    if batch.config(lanes, 1, place) != 0:
+                        assert place == qa.QT_SCRATCH_LDS
+                        continue
+                    placed.add(place)
+                    batch.launch()
+                    got, want = (t.download() for t in outs)
+                    # C of `moved`: its highest axis belongs at place mb - 1
+                    want = want.reshape(2, 1 << nb, 1 << (mb - 1)).transpose(1, 0, 2).reshape(-1)
+                    assert np.array_equal(got, want), (mb, nb, kb, a_made, b_made, lanes, place)
+            batch.close()
+    assert placed == {qa.QT_SCRATCH_LDS, qa.QT_SCRATCH_GLOBAL}
+
+
 @pytest.mark.parametrize("prec", [qa.QT_PLAIN_C128, qa.QT_C64_4M, qa.QT_C64_3M, qa.QT_C64_BF16X3])
 def test_small_programs_beside_large_ones(ctx, prec):
     """A batch without large steps runs the kernel that has no registers for them; the same
