@@ -709,8 +709,13 @@ qt_status launch_batch_t(qt_batch* b) {
     const V* pool = static_cast<const V*>(b->d_pool);
     auto d_out = reinterpret_cast<double2*>(b->d_out);
     V* const* tout = reinterpret_cast<V* const*>(b->d_tout);
+    // a batch that fits two workgroups a CU at once gains nothing from more of them, and the
+    // latency of its sums counts: a sliced run of one slice, complex128, 420 us with the LARGE
+    // instance and 430 without.  Without a sum of 16 or more the LARGE instance only has the
+    // longer code: a sweep's single slice 750 us with it, 725 without
+    const bool large = b->large_steps || (b->long_sums && b->n_inst <= 2 * b->n_cus * kExec);
 #define QT_LAUNCH_T(L, G, T)                                                                                       \
-    if (b->large_steps) {                                                                                          \
+    if (large) {                                                                                                   \
         QT_LAUNCH_M(L, G, T, true);                                                                                \
     } else {                                                                                                       \
         QT_LAUNCH_M(L, G, T, false);                                                                               \
@@ -927,6 +932,7 @@ qt_status append_programs(qt_batch* b, int n, qt_program* const* progs, const in
         for (auto st : p->steps) {
             st.tab += tab0;
             b->large_steps = b->large_steps || large_step(st);
+            b->long_sums = b->long_sums || st.k_bits >= 4;
             b->h_steps.push_back(st);
         }
         b->h_tabs.insert(b->h_tabs.end(), p->tables.begin(), p->tables.end());

@@ -107,7 +107,8 @@ struct qt_batch {
     // launch configuration
     int lanes = 64;  // 256: a workgroup per instance; 64: a wavefront; < 64: lanes per instance in a wave
     int wgs_per_cu = 4;
-    bool large_steps = false;   // a program has steps for the matrix cores, or long sums (large_step)
+    bool large_steps = false;   // a program has steps for the matrix cores or many long sums (large_step)
+    bool long_sums = false;     // a program sums 16 or more terms in a step
     bool default_shape = true;  // not chosen by qt_batch_config
     int scratch_place = QT_SCRATCH_AUTO;  // with QT_SCRATCH_STAGE_LEAVES or-ed in
     bool stage_leaves = false;
