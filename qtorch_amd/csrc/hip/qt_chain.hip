@@ -14,7 +14,6 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <vector>
 
 #include "qt_internal.h"
 #include "qt_mac.h"
@@ -335,46 +334,59 @@ __global__ __launch_bounds__(kChainThreads) void k_chain_scale(float2* __restric
     }
 }
 
-// Where a bit of the growing tensor comes from: an input position, or a bit that a step added.
-struct Origin {
-    int x;  // input position, -1: added in the chain
+// The bits of the tensor through the links, in position order: the input position each comes
+// from, -1 for a bit that a step added.
+struct Bits {
+    int n = 0;
+    int x[64];  // 40 input bits, and a step adds one at most
+
+    // summed bits (their positions ascending) taken away, `added` new ones on top
+    void step(const int* summed, int ns, int added) {
+        int m = 0;
+        for (int b = 0; b < n; ++b)
+            if (b != summed[0] && (ns < 2 || b != summed[1])) x[m++] = x[b];
+        for (int b = 0; b < added; ++b) x[m++] = -1;
+        n = m;
+    }
 };
 
-// The plan of the first n links (step_desc / step_axes as qt_contract_chain takes them), or
-// false when they cannot share a pass.
+// The plan of the first n links (desc / axes as qt_contract_chain takes them), or false when
+// they cannot share a pass.
 bool plan_chain(int nx, int dl, bool c128, int n, const int32_t* desc, const int32_t* axes, ChainPlan* out) {
-    if (n < 1 || n > kMaxLinks) return false;
+    if (n < 1 || n > kMaxLinks || nx < 1 || nx > 40) return false;
     ChainPlan p;
     std::memset(&p, 0, sizeof p);
     p.n_steps = n;
-    // bits of the tensor in position order, through the links
-    std::vector<Origin> bits(static_cast<size_t>(nx));
-    for (int i = 0; i < nx; ++i) bits[size_t(i)].x = i;
-    std::vector<char> active(size_t(nx), 0);  // input bits summed in the chain
-    std::vector<std::vector<int>> summed(static_cast<size_t>(n));  // current positions, ascending
+    Bits bits;
+    for (bits.n = 0; bits.n < nx; ++bits.n) bits.x[bits.n] = bits.n;
+    bool in_tile[64] = {false};   // input bits of the tile: first those summed in the chain
+    int summed[kMaxLinks][2];     // current positions, ascending
+    int s_x[kMaxLinks][2];        // the same in the pairs' own order
     const int32_t* ax = axes;
     for (int s = 0; s < n; ++s) {
         const int rg = desc[3 * s], k = desc[3 * s + 1], rc = desc[3 * s + 2];
-        const int rx = int(bits.size()) / dl, kb = k * dl, nb = (rg - k) * dl;
-        if (k < 1 || kb > 2 || nb < 0 || nb > 2 || k > rx || rc != rx + rg - 2 * k) return false;
+        if (k < 1 || k > 2 || rg < k || rg > k + 2) return false;
+        const int rx = bits.n / dl, kb = k * dl, nb = (rg - k) * dl;
+        if (kb > 2 || nb > 2 || k > rx || rc != rx + rg - 2 * k) return false;
         const int32_t *px = ax, *pg = ax + k, *fs = ax + 2 * k;
         ax += 2 * k + rc;
-        std::vector<char> used_x(size_t(rx), 0), used_g(size_t(rg), 0);
+        bool used_x[64] = {false}, used_g[8] = {false};
         ChainStep& st = p.step[s];
         st.ns = kb;
         st.nb = nb;
         // digit j of the summed index belongs to pair k - 1 - j (src/Network.h:912-916)
-        int s_x[2] = {0, 0}, s_g[2] = {0, 0};
+        int s_g[2] = {0, 0};
+        s_x[s][0] = s_x[s][1] = 0;
         for (int i = 0; i < k; ++i) {
-            if (px[i] < 0 || px[i] >= rx || pg[i] < 0 || pg[i] >= rg || used_x[size_t(px[i])]++ || used_g[size_t(pg[i])]++)
-                return false;
+            if (px[i] < 0 || px[i] >= rx || pg[i] < 0 || pg[i] >= rg || used_x[px[i]] || used_g[pg[i]]) return false;
+            used_x[px[i]] = used_g[pg[i]] = true;
             for (int t = 0; t < dl; ++t) {
-                s_x[(k - 1 - i) * dl + t] = px[i] * dl + t;
+                s_x[s][(k - 1 - i) * dl + t] = px[i] * dl + t;
                 s_g[(k - 1 - i) * dl + t] = pg[i] * dl + t;
             }
         }
-        for (int b = 0; b < kb; ++b) summed[size_t(s)].push_back(s_x[b]);
-        std::sort(summed[size_t(s)].begin(), summed[size_t(s)].end());
+        summed[s][0] = kb == 2 ? std::min(s_x[s][0], s_x[s][1]) : s_x[s][0];
+        summed[s][1] = kb == 2 ? std::max(s_x[s][0], s_x[s][1]) : 0;
         for (int j = 0; j < (1 << kb); ++j)
             for (int b = 0; b < kb; ++b)
                 if ((j >> b) & 1) st.g_small[j] += 1 << s_g[b];
@@ -382,96 +394,79 @@ bool plan_chain(int nx, int dl, bool c128, int n, const int32_t* desc, const int
         int prev = -1, f = 0;
         for (; f < rc && (fs[f] & QT_FROM_A); ++f) {
             const int axis = fs[f] & ~QT_FROM_A;
-            if (axis <= prev || axis >= rx || used_x[size_t(axis)]++) return false;
+            if (axis <= prev || axis >= rx || used_x[axis]) return false;
             prev = axis;
         }
         if (f != rx - k) return false;
         int g_bit[2] = {0, 0}, ng = 0;
         for (; f < rc; ++f) {
-            if ((fs[f] & QT_FROM_A) || fs[f] < 0 || fs[f] >= rg || used_g[size_t(fs[f])]++) return false;
+            if ((fs[f] & QT_FROM_A) || fs[f] < 0 || fs[f] >= rg || used_g[fs[f]]) return false;
+            used_g[fs[f]] = true;
             for (int t = 0; t < dl; ++t) g_bit[ng++] = fs[f] * dl + t;
         }
         for (int o = 0; o < (1 << nb); ++o)
             for (int b = 0; b < nb; ++b)
                 if ((o >> b) & 1) st.g_free[o] += 1 << g_bit[b];
-        // store the pairs' own order for the offsets below
-        for (int b = 0; b < kb; ++b) st.off[b] = s_x[b];
-        std::vector<Origin> next;
-        for (size_t b = 0; b < bits.size(); ++b) {
-            if (std::find(summed[size_t(s)].begin(), summed[size_t(s)].end(), int(b)) == summed[size_t(s)].end())
-                next.push_back(bits[b]);
-            else if (bits[b].x >= 0)
-                active[size_t(bits[b].x)] = 1;
-        }
-        for (int b = 0; b < nb; ++b) next.push_back(Origin{-1});
-        bits.swap(next);
+        for (int b = 0; b < kb; ++b)
+            if (bits.x[summed[s][b]] >= 0) in_tile[bits.x[summed[s][b]]] = true;
+        bits.step(summed[s], kb, nb);
     }
     // the tile: the summed input bits, the four lowest bits of the input (three in
     // complex128: 128 bytes) and of the result, then the lowest others up to the size that
     // the largest intermediate allows
     const int line = c128 ? 3 : 4;
-    std::vector<char> in_tile(active);
-    for (int i = 0; i < line && i < nx; ++i) in_tile[size_t(i)] = 1;
-    for (int i = 0; i < line && i < int(bits.size()); ++i)
-        if (bits[size_t(i)].x >= 0) in_tile[size_t(bits[size_t(i)].x)] = 1;
+    for (int i = 0; i < line && i < nx; ++i) in_tile[i] = true;
+    for (int i = 0; i < line && i < bits.n; ++i)
+        if (bits.x[i] >= 0) in_tile[bits.x[i]] = true;
     int grow = 0, most = 0;  // the largest excess of an intermediate over the input tile
     for (int s = 0; s < n; ++s) {
         grow += p.step[s].nb - p.step[s].ns;
         most = std::max(most, grow);
     }
     int tb = 0;
-    for (char t : in_tile) tb += t;
+    for (int i = 0; i < nx; ++i) tb += in_tile[i];
     // at least 2^8 tiles where the tensor is small, and a tile that fills the workgroup
     const int cap = std::min(c128 ? kMaxTileBits - 1 : kMaxTileBits, std::max(9, nx - 8));
     if (tb + most > cap || tb + grow < 2) return false;
     for (int i = 0; i < nx && tb + most < cap; ++i)
-        if (!in_tile[size_t(i)]) {
-            in_tile[size_t(i)] = 1;
+        if (!in_tile[i]) {
+            in_tile[i] = true;
             ++tb;
         }
     p.tb_in = tb;
     p.tb_out = tb + grow;
     int k = 0;
     for (int i = 0; i < nx; ++i)
-        if (in_tile[size_t(i)]) p.in_pos[k++] = i;
+        if (in_tile[i]) p.in_pos[k++] = i;
     k = 0;
     int r = 0;
-    for (size_t i = 0; i < bits.size(); ++i) {
-        if (bits[i].x < 0 || in_tile[size_t(bits[i].x)]) {
-            p.out_pos[k++] = int(i);
+    for (int i = 0; i < bits.n; ++i) {
+        if (bits.x[i] < 0 || in_tile[bits.x[i]]) {
+            p.out_pos[k++] = i;
         } else {
-            p.rest_in[r] = bits[i].x;
-            p.rest_out[r++] = int(i);
+            p.rest_in[r] = bits.x[i];
+            p.rest_out[r++] = i;
         }
     }
     p.n_rest = r;
     if (k != p.tb_out || r > 48) return false;
     // tile positions of the summed bits: their rank among the tile's bits at that step
-    std::vector<Origin> cur(static_cast<size_t>(nx));
-    for (int i = 0; i < nx; ++i) cur[size_t(i)].x = i;
+    Bits cur;
+    for (cur.n = 0; cur.n < nx; ++cur.n) cur.x[cur.n] = cur.n;
     for (int s = 0; s < n; ++s) {
         ChainStep& st = p.step[s];
-        std::vector<int> rank_of(cur.size(), -1);
-        int lb = 0;
-        for (size_t b = 0; b < cur.size(); ++b)
-            if (cur[b].x < 0 || in_tile[size_t(cur[b].x)]) rank_of[b] = lb++;
+        int rank_of[64], lb = 0;
+        for (int b = 0; b < cur.n; ++b) rank_of[b] = cur.x[b] < 0 || in_tile[cur.x[b]] ? lb++ : -1;
         st.lb = lb;
         if (lb - st.ns < 1) return false;  // a thread takes two free parts
-        const int s_x[2] = {st.off[0], st.off[1]};
         st.adj = -1;
         for (int b = 0; b < st.ns; ++b)
-            if (rank_of[size_t(s_x[b])] == 0) st.adj = b;
-        for (int i = 0; i < st.ns; ++i) st.ins[i] = rank_of[size_t(summed[size_t(s)][size_t(i)])];
-        std::memset(st.off, 0, sizeof st.off);
+            if (rank_of[s_x[s][b]] == 0) st.adj = b;
+        for (int i = 0; i < st.ns; ++i) st.ins[i] = rank_of[summed[s][i]];
         for (int j = 0; j < (1 << st.ns); ++j)
             for (int b = 0; b < st.ns; ++b)
-                if ((j >> b) & 1) st.off[j] += 1 << rank_of[size_t(s_x[b])];
-        std::vector<Origin> next;
-        for (size_t b = 0; b < cur.size(); ++b)
-            if (std::find(summed[size_t(s)].begin(), summed[size_t(s)].end(), int(b)) == summed[size_t(s)].end())
-                next.push_back(cur[b]);
-        for (int b = 0; b < st.nb; ++b) next.push_back(Origin{-1});
-        cur.swap(next);
+                if ((j >> b) & 1) st.off[j] += 1 << rank_of[s_x[s][b]];
+        cur.step(summed[s], st.ns, st.nb);
     }
     *out = p;
     return true;

@@ -254,6 +254,61 @@ SlicedNetwork::SlicedNetwork(const std::string& qasm, const std::string& measure
         leaf_rank_[size_t(i)] = r;
     }
     PlanFusion();
+    PlanPasses(!roots_.empty());
+}
+
+int64_t SlicedNetwork::PlanPasses(bool fuse) {
+    constexpr size_t kMost = 8;  // links of one pass
+    const int n = int(steps_.size());
+    auto& forms = passes_[fuse ? 1 : 0];
+    forms.assign(kPassForms, Passes());
+    // results alive before each step, in the order of the plan
+    auto bytes = [&](int step) { return int64_t(16) << (steps_[size_t(step)].rank_c * dl_); };
+    std::vector<int64_t> live(size_t(n) + 1, 0);
+    for (int s = 0; s < n; ++s) {
+        live[size_t(s) + 1] = live[size_t(s)] + bytes(s);
+        for (int op : {steps_[size_t(s)].a, steps_[size_t(s)].b})
+            if (op >= n_leaves_) live[size_t(s) + 1] -= bytes(op - n_leaves_);
+    }
+    int64_t peak = 0;
+    for (int form = 0; form < kPassForms; ++form) {
+        Passes& p = forms[size_t(form)];
+        p.at.assign(size_t(n), -1);
+        const int dtype = form == kPassC128 ? QT_DTYPE_C128 : QT_DTYPE_C64;
+        for (int s = 0; s < n; ++s) {
+            if (fuse && step_fused_[size_t(s)]) continue;
+            // consecutive steps that each contract the last result (as operand A) with
+            // another tensor; a rescaled run's own results carry exponents, which a pass
+            // does not take from the small tensors (leaves and subtrees have none)
+            Pass pass;
+            for (int q = s; q < n && pass.links.size() < kMost; ++q) {
+                if (fuse && step_fused_[size_t(q)]) continue;
+                const Step& l = steps_[size_t(q)];
+                if (!pass.links.empty() && l.a != n_leaves_ + pass.links.back()) break;
+                if (form == kPassC64Rescaled && l.b >= n_leaves_ && !(fuse && step_fused_[size_t(l.b - n_leaves_)]))
+                    break;
+                pass.links.push_back(q);
+                pass.desc.insert(pass.desc.end(), {l.rank_b, l.k, l.rank_c});
+                pass.axes.insert(pass.axes.end(), l.pair_a.begin(), l.pair_a.end());
+                pass.axes.insert(pass.axes.end(), l.pair_b.begin(), l.pair_b.end());
+                pass.axes.insert(pass.axes.end(), l.free_src.begin(), l.free_src.end());
+            }
+            if (pass.links.size() < 2) continue;
+            const int taken = qt_chain_links(steps_[size_t(s)].rank_a, dl_, dtype, int(pass.links.size()),
+                                             pass.desc.data(), pass.axes.data());
+            if (taken < 2) continue;
+            pass.links.resize(size_t(taken));
+            const int last = pass.links.back();
+            int64_t during = live[size_t(s)] + bytes(last);
+            for (int q : pass.links)
+                if (steps_[size_t(q)].b >= n_leaves_ + s) during += bytes(steps_[size_t(q)].b - n_leaves_);
+            peak = std::max(peak, during);
+            p.at[size_t(s)] = int(p.all.size());
+            p.all.push_back(std::move(pass));
+            s = last;
+        }
+    }
+    return peak;
 }
 
 // Small steps (result <= 2^12 elements, operands <= 2^14, <= 2^16 complex MACs) whose
@@ -610,6 +665,8 @@ std::complex<double> SlicedNetwork::RunWith(qt_ctx* ctx, int precision, SliceSta
         std::vector<const void*> ptrs(direct.size());
         std::vector<qt_tensor*> made(direct.size());
         std::vector<double> block;
+        std::vector<const qt_tensor*> small;  // of one pass
+        const Passes& passes = passes_[fuse ? 1 : 0][c128 ? kPassC128 : base == precision ? kPassC64 : kPassC64Rescaled];
         // the slices contracted: the list, else the range (every slice by default)
         const bool listed = !slice_list_.empty();
         const int64_t s_begin = listed ? 0 : slice_first_;
@@ -677,45 +734,26 @@ std::complex<double> SlicedNetwork::RunWith(qt_ctx* ctx, int precision, SliceSta
                 for (size_t s = 0; s < steps_.size(); ++s) {
                     if (fuse && step_fused_[s]) continue;
                     const Step& st = steps_[s];
-                    // consecutive steps that each contract the last result (as operand A)
-                    // with another tensor: as many as one pass takes
-                    std::vector<size_t> link{s};
-                    for (size_t q = s + 1; q < steps_.size() && link.size() < 8; ++q) {
-                        if (fuse && step_fused_[q]) continue;
-                        if (steps_[q].a != n_leaves_ + int(link.back()) || !ops[size_t(steps_[q].b)]) break;
-                        link.push_back(q);
-                    }
-                    int taken = 0;
-                    std::vector<int32_t> desc, axes;
-                    if (link.size() > 1) {
-                        for (size_t q : link) {
-                            const Step& l = steps_[q];
-                            desc.insert(desc.end(), {l.rank_b, l.k, l.rank_c});
-                            axes.insert(axes.end(), l.pair_a.begin(), l.pair_a.end());
-                            axes.insert(axes.end(), l.pair_b.begin(), l.pair_b.end());
-                            axes.insert(axes.end(), l.free_src.begin(), l.free_src.end());
-                        }
-                        taken = qt_chain_links(st.rank_a, dl_, dtype, int(link.size()), desc.data(), axes.data());
-                    }
+                    const Pass* pass = passes.at[s] >= 0 ? &passes.all[size_t(passes.at[s])] : nullptr;
                     qt_tensor* c = nullptr;
-                    if (taken > 0) {
-                        link.resize(size_t(taken));
-                        std::vector<const qt_tensor*> small;
-                        for (size_t q : link) small.push_back(ops[size_t(steps_[q].b)]);
-                        CheckQt(ctx, qt_tensor_alloc_empty(ctx, steps_[link.back()].rank_c, dl_, dtype, &c),
-                                "qt_tensor_alloc_empty");
-                        const qt_status got = qt_contract_chain(ctx, ops[size_t(st.a)], st.rank_a, taken, small.data(),
-                                                                desc.data(), axes.data(), c, precision);
-                        if (got == QT_UNSUPPORTED) {  // a small tensor with an exponent: step by step
-                            qt_tensor_free(ctx, c);
-                            taken = 0;
+                    if (pass) {
+                        small.clear();
+                        for (int q : pass->links) small.push_back(ops[size_t(steps_[size_t(q)].b)]);
+                        const int last = pass->links.back();
+                        qt_status got = qt_tensor_alloc_empty(ctx, steps_[size_t(last)].rank_c, dl_, dtype, &c);
+                        if (got == QT_OK)
+                            got = qt_contract_chain(ctx, ops[size_t(st.a)], st.rank_a, int(small.size()), small.data(),
+                                                    pass->desc.data(), pass->axes.data(), c, precision);
+                        if (got == QT_OOM) {  // no room beside the operands: step by step
+                            if (c) qt_tensor_free(ctx, c);
+                            c = nullptr;
+                            pass = nullptr;
                         } else {
-                            ops[size_t(n_leaves_) + link.back()] = c;
+                            ops[size_t(n_leaves_ + last)] = c;
                             CheckQt(ctx, got, "qt_contract_chain");
                         }
                     }
-                    if (taken == 0) {
-                        link.resize(1);
+                    if (!pass) {
                         CheckQt(ctx, qt_tensor_alloc_empty(ctx, st.rank_c, dl_, dtype, &c), "qt_tensor_alloc_empty");
                         ops[size_t(n_leaves_) + s] = c;
                         CheckQt(ctx,
@@ -729,8 +767,12 @@ std::complex<double> SlicedNetwork::RunWith(qt_ctx* ctx, int precision, SliceSta
                         ops[size_t(op)] = nullptr;
                     };
                     done(st.a);
-                    for (size_t q : link) done(steps_[q].b);
-                    s = link.back();
+                    if (!pass) {
+                        done(st.b);
+                        continue;
+                    }
+                    for (int q : pass->links) done(steps_[size_t(q)].b);
+                    s = size_t(pass->links.back());
                 }
                 CheckQt(ctx, qt_tensor_accumulate(ctx, ops.back(), acc), "qt_tensor_accumulate");
                 release();

@@ -49,7 +49,10 @@ public:
     const SliceStats& Plan() const { return plan_; }
     // slices_per_launch = 0: every step through qt_contract_pair; < 0 (default): fused
     // subtrees, slices per launch chosen by memory; > 0: at most that many per launch.
-    void SetFusion(int64_t slices_per_launch) { fuse_slices_ = slices_per_launch; }
+    void SetFusion(int64_t slices_per_launch) {
+        fuse_slices_ = slices_per_launch;
+        if (slices_per_launch == 0 && passes_[0].empty()) PlanPasses(false);
+    }
     // Run contracts only slices [first, first + count) of the plan's slices (count < 0:
     // to the last one) and returns their sum; the default is every slice.
     void SetSliceRange(int64_t first, int64_t count);
@@ -75,7 +78,21 @@ private:
         int rank_a, rank_b, k, rank_c;
         std::vector<int32_t> pair_a, pair_b, free_src;
     };
+    // Consecutive steps that qt_contract_chain runs in one pass (they depend on the
+    // structure only, so they are planned once and not in every slice).
+    struct Pass {
+        std::vector<int> links;  // the steps, each contracting the last one's result
+        std::vector<int32_t> desc, axes;
+    };
+    struct Passes {
+        std::vector<Pass> all;
+        std::vector<int> at;  // per step: the pass it begins, or -1
+    };
+    enum { kPassC128, kPassC64, kPassC64Rescaled, kPassForms };
     void PlanFusion();
+    // The passes of fused or unfused runs; returns the bytes (complex128) of a slice's live
+    // results while the largest of them runs.
+    int64_t PlanPasses(bool fuse);
     // leaf i's sub-tensor for `slice` as interleaved FP64 (re, im) at dst
     void Extract(int leaf, int64_t slice, double* dst) const { Extract(leaf_vals_, leaf, slice, dst); }
     void Extract(const std::vector<std::vector<std::complex<double>>>& vals, int leaf, int64_t slice,
@@ -100,6 +117,7 @@ private:
     int64_t fuse_slices_ = -1;
     int64_t slice_first_ = 0, slice_count_ = -1;
     std::vector<int64_t> slice_list_;  // non-empty: the slices Run contracts
+    std::vector<Passes> passes_[2];                 // of unfused and fused runs, by kPass form
     std::vector<char> step_fused_;                  // per step
     std::vector<char> leaf_direct_;                 // per leaf: an operand of an unfused step
     std::vector<int> roots_;                        // root step of each subtree

@@ -189,3 +189,19 @@ def test_sweep_with_chains_matches_line_graph(ctx):
     for prec, tol in ((qa.QT_PLAIN_C128, 1e-11), (qa.QT_C64_4M, 2e-5), (qa.QT_C64_4M | qa.QT_RESCALE, 2e-5)):
         v, _ = sweep.run(ctx, prec)
         assert abs(v - ref) <= tol * max(abs(ref), 2.0 ** -10)
+
+
+@pytest.mark.parametrize("order,fusion", [(qa.ORDER_SWEEP, 0), (qa.ORDER_LINEGRAPH, 0), (qa.ORDER_LINEGRAPH, -1)])
+def test_runs_take_only_passes_that_fit(order, fusion):
+    """Rescaled runs with small tensors that carry exponents (every unfused result does): no
+    pass is tried and refused, which would leave its message on the context."""
+    ctx = qa.Context(0)
+    q, bits = wl.grid_random_circuit(4, 5, 14, seed=3), wl.bitstring(20, 4)
+    net = qa.SlicedNetwork(q, bits, dim_log2=1, order=order, max_bits=28)
+    ref, _ = net.run(ctx)
+    net.set_fusion(fusion)
+    v, _ = net.run(ctx, qa.QT_C64_4M | qa.QT_RESCALE)
+    assert abs(v - ref) <= 2e-5 * max(abs(ref), 2.0 ** -10)
+    assert hip.qt_last_error(ctx.handle) == b""
+    net.close()
+    ctx.close()
