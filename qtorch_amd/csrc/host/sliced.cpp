@@ -254,7 +254,8 @@ SlicedNetwork::SlicedNetwork(const std::string& qasm, const std::string& measure
         leaf_rank_[size_t(i)] = r;
     }
     PlanFusion();
-    PlanPasses(!roots_.empty());
+    const int64_t pass_peak = PlanPasses(!roots_.empty());
+    if (pass_peak > peak) plan_.peak_bytes += pass_peak - peak;
 }
 
 int64_t SlicedNetwork::PlanPasses(bool fuse) {
@@ -408,6 +409,16 @@ void SlicedNetwork::PlanFusion() {
         const int64_t chunk = std::max<int64_t>(
             1, std::min<int64_t>({plan_.slices, 4096, (int64_t(256) << 20) / std::max<int64_t>(1, root_bytes_c128_)}));
         plan_.peak_bytes += chunk * (root_bytes_c128_ + 16 * block_elems_) + int64_t(const_pool_.size()) * 8;
+        // their executors' scratch, where it does not fit LDS (more than 64 KiB each): one
+        // area per workgroup of the grid, at least one and at most four a CU, 4 GiB in all
+        int64_t scratch = 0;
+        for (const auto& p : progs_) {
+            int64_t elems = 0;
+            (void)qt_program_stats(p.get(), nullptr, &elems, nullptr);
+            scratch = std::max(scratch, 16 * ((elems + 15) / 16 * 16));
+        }
+        const int64_t wgs = std::max<int64_t>(256, std::min<int64_t>(1024, chunk * int64_t(roots_.size())));
+        if (scratch > 64 * 1024) plan_.peak_bytes += std::min<int64_t>(int64_t(4) << 30, wgs * scratch);
     }
 }
 

@@ -494,6 +494,23 @@ def test_sliced_planned_bytes_cover_step_scratch():
     assert plan["peak_bytes"] >= need + (64 << 20), (plan["peak_bytes"], need)
 
 
+def test_sliced_planned_bytes_cover_passes_and_programs():
+    """Planned device bytes cover a pass's operand and result, which live at once (both of the
+    largest size in this sweep), and the scratch of the fused programs' executors: one area
+    for each of 256 workgroups at least, where a program's intermediates exceed 64 KiB."""
+    from qtorch_amd import workloads as wl
+    sweep = qa.SlicedNetwork(wl.grid_random_circuit(4, 5, 14, seed=5), wl.bitstring(20, 1), dim_log2=1,
+                             order=qa.ORDER_SWEEP, max_bits=29).plan()
+    assert sweep["peak_bytes"] >= (64 << 20) + 2 * (16 << sweep["peak_bits"])
+    q, bits = wl.grid_random_circuit(3, 5, 8, seed=5), wl.bitstring(15, 1)
+    plan = qa.SlicedNetwork(q, bits, dim_log2=1, order=qa.ORDER_LINEGRAPH, max_bits=28).plan()
+    net = qa.Network(q, bits, dim_log2=1)
+    net.order(qa.ORDER_LINEGRAPH, 0)
+    stats = net.program_stats()  # every step is in one fused program
+    assert plan["fused_steps"] == stats["n_steps"] and 16 * stats["scratch_elems"] > 64 << 10
+    assert plan["peak_bytes"] >= (64 << 20) + 256 * 16 * stats["scratch_elems"]
+
+
 def test_nonzero_slices_report_a_truncated_search():
     """qth_sliced_nonzero_slices_ex: a budget too small to finish says so (complete =
     0); a sufficient one lists every nonzero slice and says it is complete; the plain
