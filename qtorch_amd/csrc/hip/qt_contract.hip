@@ -308,9 +308,11 @@ __device__ __forceinline__ V shfl_xor_v(V v, int d) {
 // next log2(gridDim.x) bits) and the step (the bits above).  The host orders the summed
 // bits (order_summed_bits): the lanes of a wave cover the lowest summed bits of A and of
 // B in turn, so that both operands are read in whole 64-byte pieces however their axes
-// lie, and workgroups that run together read neighbouring runs.  Every output is summed
-// in the same order whatever the grouping: each lane over its steps in order, then the
-// lanes of a wave pairwise (lane bits 5 to 0), then the waves in order.
+// lie, and workgroups that run together read neighbouring runs.  Every output of a call is
+// summed in the same fixed order: each lane over its steps in order, then the lanes of a
+// wave pairwise (lane bits 5 to 0), the waves in order, the workgroups in order.  How many
+// steps a workgroup takes depends on the number of row groups (run_reduce), so the order
+// differs between shapes, and from the one-output-per-lane kernels'.
 // Bound by HBM.  A step of two complex64 operands (2^25 and 2^24 elements, shuffled axes,
 // 8 x 4 outputs, 2^22 summed indices: 403 MB), read-back included: 119 us, 586 us with
 // the lanes on the pairs' own bit order and two passes of 4 x 4 outputs.
@@ -1289,9 +1291,9 @@ namespace {
 
 // Large complex64 GEMMs in the 4M / 3M forms: 128x128 output tile per workgroup,
 // four waves of 64x64 (4x4 blocks of v_mfma_f32_16x16x4f32), k-tiles of 16; the next
-// k-tile is loaded into registers while the current one is multiplied from LDS.
-// LDS rows are 144 floats apart, so the four k-rows a wave reads at once sit in
-// different bank quarters.
+// k-tile is staged in a second LDS buffer while the current one is multiplied.
+// LDS rows are 144 complex values apart (288 words: half of the 64 banks beyond whole
+// turns), so the two k-rows that half a wave reads at once sit in different halves.
 constexpr int BT = 128, BK = 16, BROW = BT + 16;
 constexpr int64_t kSplitRows = 256;
 

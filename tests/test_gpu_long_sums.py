@@ -33,7 +33,7 @@ SHAPES = [(0, 0, 9, 1), (0, 3, 10, 1), (11, 0, 9, 1), (5, 6, 9, 1), (2, 3, 5, 2)
           (12, 0, 11, 1), (1, 11, 11, 1), (10, 6, 11, 1), (0, 8, 6, 2), (4, 3, 12, 1)]
 
 
-@pytest.mark.parametrize("prec,tol", [(qa.QT_PLAIN_C128, 0.0), (qa.QT_C64_4M, 2e-6), (qa.QT_C64_3M, 4e-6),
+@pytest.mark.parametrize("prec,tol", [(qa.QT_PLAIN_C128, 1e-13), (qa.QT_C64_4M, 2e-6), (qa.QT_C64_3M, 4e-6),
                                       (qa.QT_C64_BF16X3, 1e-4)])
 @pytest.mark.parametrize("fa,fb,k,d", SHAPES)
 def test_long_sums(ctx, fa, fb, k, d, prec, tol):
@@ -53,8 +53,7 @@ def test_long_sums(ctx, fa, fb, k, d, prec, tol):
         got = qa.contract_pair(ctx, ta, tb, pairs, free, prec)[0].download()
         ref = _tensordot(a, ra, b, rb, free, pairs, d)
         # sums of 2^(d k) products of unit variance: rounding of about sqrt(2^(d k)) terms
-        bound = 1e-13 if c128 else tol
-        assert np.abs(got - ref).max() <= bound * np.sqrt(1 << (d * k)) * max(np.abs(ref).max(), 1.0)
+        assert np.abs(got - ref).max() <= tol * np.sqrt(1 << (d * k)) * max(np.abs(ref).max(), 1.0)
 
 
 def test_long_sum_without_room_for_partial_sums():

@@ -64,7 +64,7 @@ def _regime(free, k, d):
     nc, ns = len(free) * d, k * d
     if split and na * d >= 6 and (len(free) - na) * d >= 6 and (ns >= 4 or (ns >= 3 and nc >= 24)):
         return "gemm"
-    if nc <= 6 and ns >= 13:
+    if (ns >= 11 and nc <= 16) or (ns >= 9 and nc <= 11):
         return "reduce"
     if split and min(na * d, nc - na * d) <= 5 and max(na * d, nc - na * d) >= 10:
         return "skinny"

@@ -1,6 +1,7 @@
 """GPU tests of qt_contract_pair_noalloc, the entry point that allocates nothing: its
 scratch is a fixed 64 MiB device array per GPU.  Through the C ABI, against
-qt_contract_pair on the same tensors (the same kernels: identical bits), two calls
+qt_contract_pair on the same tensors (identical bits where both take the same kernels,
+rounding apart where only qt_contract_pair splits a long sum), two calls
 in a row with the second smaller, in the GEMM regime (operand permutes in the
 array) and the split reduction (partial sums in the array); steps whose scratch
 exceeds the array, and QT_RESCALE, are refused before anything runs."""
@@ -75,6 +76,24 @@ def test_noalloc_equals_contract_pair(ctx, seq):
         if dt == qa.QT_DTYPE_C128 and ra + rb <= 16:  # and the oracle, where it is quick
             o = qo.contract_indices(a_h, ra, b_h, rb, free, pairs, dim_log2=d)
             assert np.allclose(got, o, rtol=1e-12, atol=1e-12 * np.abs(o).max())
+
+
+@pytest.mark.parametrize("dt", [qa.QT_DTYPE_C128, qa.QT_DTYPE_C64])
+@pytest.mark.parametrize("ra,rb,k", [(12, 20, 12), (9, 20, 9), (16, 20, 12)])
+def test_noalloc_long_sums(ctx, ra, rb, k, dt):
+    """2^12 terms into 2^8 and 2^12 outputs, 2^9 into 2^11: split by qt_contract_pair, one
+    output a lane here (no scratch); both against numpy in complex128."""
+    rng = np.random.default_rng(ra + rb)
+    npdt, prec = (np.complex128, qa.QT_PLAIN_C128) if dt == qa.QT_DTYPE_C128 else (np.complex64, qa.QT_C64_4M)
+    pairs = [(i, i) for i in range(k)]
+    free = [(True, i) for i in range(k, ra)] + [(False, j) for j in range(k, rb)]
+    a_h, b_h = _rand(rng, 1 << ra, npdt), _rand(rng, 1 << rb, npdt)
+    a, b = (qa.Tensor(ctx, r, 1, dt).upload(x) for r, x in ((ra, a_h), (rb, b_h)))
+    ref = (b_h.astype(np.complex128).reshape(-1, 1 << k) @ a_h.astype(np.complex128).reshape(-1, 1 << k).T).reshape(-1)
+    # 2^k products of unit variance, each sum rounded about 2^k times at up to its own size
+    bound = (1e-15 if dt == qa.QT_DTYPE_C128 else 6e-7) * 2 ** k
+    for c in (qa.contract_pair(ctx, a, b, pairs, free, prec)[0], _noalloc(ctx, a, b, pairs, free, prec)[0]):
+        assert np.abs(c.download() - ref).max() <= bound
 
 
 def test_noalloc_refuses_what_does_not_fit(ctx):
